@@ -1,0 +1,407 @@
+"""Performance cases: the work that a program using this package has it do.
+
+Each case is one call through a public entry point on tensors that are already
+on the GPU, as a decode or prefill loop makes it:
+
+  matvec     device.QMat.matvec            one vector (decode), or a few (speculative tokens, small batches)
+  matmul     device.QMat.matmul            prefill product with a quantized matrix
+  chain      layer.DecodeLayerChain        the seven matvecs of a decode layer with norms, SiLU*up, residuals, RoPE
+  moe        moe.MoELayer.forward_device   top-k MoE layer, one token to a prefill batch
+  attention  attention.attention_decode    grouped-query attention of one token over the KV cache
+
+Weights are seeded GGML blocks with the distributions of localai_amd.synth
+(uniform quants and sub-block scales, fp16 block scales), activations N(0, 1).
+GGML type numbers: 2 Q4_0, 8 Q8_0, 12 Q4_K, 13 Q5_K, 14 Q6_K.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+from localai_amd import attention, device, layer, moe
+
+# type -> (values per block, bytes per block)
+LAYOUT = {2: (32, 18), 8: (32, 34), 12: (256, 144), 13: (256, 176), 14: (256, 210)}
+# type -> (offsets of the fp16 scales, their range)
+SCALES = {2: ((0,), (1e-4, 2e-3)), 8: ((0,), (1e-4, 1e-2)), 12: ((0, 2), (1e-4, 2e-3)),
+          13: ((0, 2), (1e-4, 2e-3)), 14: ((208,), (1e-4, 2e-3))}
+EPS = 1e-5
+# the costliest listed prefill product, which drawn ones do not exceed
+MOST_PRODUCTS = 14336 * 4096 * 2048
+
+
+def _matvec(name, t, rows, cols, tokens):
+    return {'name': name, 'kind': 'matvec', 'type': t, 'rows': rows, 'cols': cols, 'tokens': tokens}
+
+
+def _matmul(name, t, rows, cols, tokens):
+    return {'name': name, 'kind': 'matmul', 'type': t, 'rows': rows, 'cols': cols, 'tokens': tokens}
+
+
+def _moe(name, t, experts, hidden, inter, top_k, tokens, zipf):
+    return {'name': name, 'kind': 'moe', 'type': t, 'experts': experts, 'hidden': hidden, 'inter': inter,
+            'top_k': top_k, 'tokens': tokens, 'zipf': zipf}
+
+
+def listed():
+    return [
+        # one token through Llama-3-8B's attn_k: the smallest matrix of a decode step, called once per layer
+        _matvec('matvec_attn_k_q4_k', 12, 1024, 4096, 1),
+        # seven drafted tokens checked together (or seven sequences decoded together) through ffn_gate
+        _matvec('matvec_ffn_gate_q4_k_t7', 12, 14336, 4096, 7),
+        # Llama-3-8B's vocabulary head, once per generated token
+        _matvec('matvec_vocab_head_q6_k', 14, 128256, 4096, 1),
+        # a Llama-3-8B decode layer after its attention, Q4_K_M types: what a decode step consists of
+        {'name': 'chain_llama3_8b', 'kind': 'chain', 'dim': 4096, 'ffn': 14336, 'head_dim': 128, 'kv_heads': 8},
+        # a short chat turn of odd length through attn_q / attn_output
+        _matmul('matmul_attn_q_q4_k_t77', 12, 4096, 4096, 77),
+        # a chat turn through the ffn_up of a Q5_K_M file
+        _matmul('matmul_ffn_up_q5_k_t128', 13, 14336, 4096, 128),
+        # a longer, odd prompt through ffn_down, the long rows of a layer (Q6_K in a Q4_K_M file)
+        _matmul('matmul_ffn_down_q6_k_t333', 14, 4096, 14336, 333),
+        # a 512-token prefill chunk of a Q8_0 file (the benchmark's prefill shape)
+        _matmul('matmul_ffn_gate_q8_0_t512', 8, 14336, 4096, 512),
+        # a 2048-token document through ffn_gate: the largest call
+        _matmul('matmul_ffn_gate_q4_k_t2048', 12, 14336, 4096, 2048),
+        # one decode token of ZAYA's MoE layer
+        _moe('moe_zaya_q6_k_t1', 14, 16, 2048, 4096, 2, 1, False),
+        # a 512-token prefill chunk of a Qwen3-MoE layer, experts unevenly popular
+        _moe('moe_qwen3_q4_k_t512', 12, 128, 2048, 768, 8, 512, True),
+        # a Llama-3-8B head set over a 4096-token conversation
+        {'name': 'attention_llama3_8b_4096', 'kind': 'attention', 'heads': 32, 'kv_heads': 8, 'head_dim': 128,
+         'position': 4095, 'window': 0, 'gate': False},
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(['matvec', 'matmul', 'matmul', 'matmul', 'moe', 'chain', 'attention'])
+    t = rng.choice([2, 8, 12, 12, 13, 14])
+    if kind in ('matvec', 'matmul'):
+        rows = _log(rng, 512, 32000)
+        if rng.random() < 0.7:
+            rows = max(256, rows // 256 * 256)
+        cols = 256 * _log(rng, 4, 56)
+        if kind == 'matvec':
+            tokens = rng.choice([1, _log(rng, 2, 31)])
+            return {'kind': kind, 'type': t, 'rows': rows, 'cols': cols, 'tokens': tokens}
+        tokens = max(32, min(_log(rng, 32, 2048), MOST_PRODUCTS // (rows * cols)))
+        return {'kind': kind, 'type': t, 'rows': rows, 'cols': cols, 'tokens': tokens}
+    if kind == 'moe':
+        # ZAYA, Qwen3-MoE and Mixtral-like layers
+        experts, hidden, inter, top_k, t = rng.choice([(16, 2048, 4096, 2, 14), (128, 2048, 768, 8, 12),
+                                                       (8, 4096, 14336, 2, 12), (64, 2048, 1024, 6, 12)])
+        most = 512 if inter < 4096 else 128
+        return {'kind': kind, 'type': t, 'experts': experts, 'hidden': hidden, 'inter': inter, 'top_k': top_k,
+                'tokens': _log(rng, 1, most), 'zipf': rng.random() < 0.5}
+    if kind == 'chain':
+        dim = 512 * rng.randint(4, 10)
+        return {'kind': kind, 'dim': dim, 'ffn': 256 * rng.randint(2 * dim // 256, 14336 // 256), 'head_dim': 128,
+                'kv_heads': rng.choice([4, 8])}
+    head_dim, per = rng.choice([(64, 4), (64, 8), (128, 4), (128, 8), (256, 2), (256, 4)])
+    kv_heads = rng.choice([2, 4, 8])
+    return {'kind': kind, 'heads': kv_heads * per, 'kv_heads': kv_heads, 'head_dim': head_dim,
+            'position': _log(rng, 16, 16384), 'window': rng.choice([0, 0, 1024]), 'gate': rng.random() < 0.3}
+
+
+# ---- inputs ------------------------------------------------------------------
+
+def _dev():
+    return device.device()
+
+
+def _gen(seed):
+    g = torch.Generator(device=_dev())
+    g.manual_seed(int(seed))
+    return g
+
+
+def _ggml(g, t, values):
+    """Seeded GGML blocks as a [blocks, bytes] uint8 device tensor."""
+    block, size = LAYOUT[t]
+    n = values // block
+    b = torch.randint(0, 256, (n, size), dtype=torch.uint8, device=_dev(), generator=g)
+    if t == 8:
+        b[:, 2:] = torch.randint(-127, 128, (n, 32), dtype=torch.int8, device=_dev(), generator=g).view(torch.uint8)
+    offs, (lo, hi) = SCALES[t]
+    for o in offs:
+        d = lo + (hi - lo) * torch.rand((n, 1), device=_dev(), generator=g)
+        b[:, o:o + 2] = d.to(torch.float16).view(torch.uint8)
+    return b
+
+
+def _normal(g, *shape):
+    return torch.randn(shape, dtype=torch.float32, device=_dev(), generator=g)
+
+
+def _chain_shapes(c):
+    kv = c['kv_heads'] * c['head_dim']
+    return {'attn_output': (12, c['dim'], c['dim']), 'ffn_gate': (12, c['ffn'], c['dim']),
+            'ffn_up': (12, c['ffn'], c['dim']), 'ffn_down': (14, c['dim'], c['ffn']),
+            'attn_q': (12, c['dim'], c['dim']), 'attn_k': (12, kv, c['dim']), 'attn_v': (14, kv, c['dim'])}
+
+
+def _inputs(c, seed):
+    """The case's data, from the seed alone."""
+    g = _gen(seed)
+    kind = c['kind']
+    if kind in ('matvec', 'matmul'):
+        raw = _ggml(g, c['type'], c['rows'] * c['cols'])
+        x = _normal(g, c['tokens'], c['cols'])
+        return {'raw': raw, 'x': x}
+    if kind == 'chain':
+        raws = {n: _ggml(g, t, r * k) for n, (t, r, k) in _chain_shapes(c).items()}
+        half = c['head_dim'] // 2
+        angle = 1000.0 * 500000.0 ** (-torch.arange(half, device=_dev(), dtype=torch.float64) / half)
+        return {'raws': raws, 'pre': _normal(g, c['dim']), 'att': _normal(g, c['dim']),
+                'w_ffn': 1.0 + 0.1 * _normal(g, c['dim']), 'w_attn': 1.0 + 0.1 * _normal(g, c['dim']),
+                'cos': torch.cos(angle).float(), 'sin': torch.sin(angle).float()}
+    if kind == 'moe':
+        e, h, i = c['experts'], c['hidden'], c['inter']
+        router = 0.02 * _normal(g, e, h)
+        bias = None
+        if c['zipf']:
+            p = torch.arange(1, e + 1, device=_dev(), dtype=torch.float64) ** -1.1
+            bias = torch.log(p / p.sum()).float()
+        return {'router': router, 'bias': bias, 'gate_up': _ggml(g, c['type'], e * 2 * i * h),
+                'down': _ggml(g, c['type'], e * h * i), 'h': _normal(g, c['tokens'], h)}
+    nh, nkv, hd, n = c['heads'], c['kv_heads'], c['head_dim'], c['position'] + 1
+    return {'k': _normal(g, n, nkv, hd), 'v': _normal(g, n, nkv, hd), 'q': _normal(g, nh * hd),
+            'k_new': _normal(g, nkv * hd), 'v_new': _normal(g, nkv * hd),
+            'gate': _normal(g, nh * hd) if c['gate'] else None}
+
+
+def _max_seq(c):
+    return max(256, 1 << c['position'].bit_length())
+
+
+def prepare(case, seed):
+    c, d = case, _inputs(case, seed)
+    kind = c['kind']
+    if kind in ('matvec', 'matmul'):
+        q = device.QMat.from_ggml(d['raw'], c['type'], c['rows'], c['cols'])
+        x = d['x'].reshape(-1) if kind == 'matvec' and c['tokens'] == 1 else d['x']
+        return {'kind': kind, 'q': q, 'x': x}
+    if kind == 'chain':
+        mats = {n: device.QMat.from_ggml(d['raws'][n], t, r, k) for n, (t, r, k) in _chain_shapes(c).items()}
+        ch = layer.DecodeLayerChain(mats, d['w_ffn'].cpu().numpy(), d['w_attn'].cpu().numpy(), EPS, c['head_dim'])
+        return {'kind': kind, 'chain': ch, 'pre': d['pre'], 'att': d['att'], 'rope': (d['cos'], d['sin'])}
+    if kind == 'moe':
+        bias = None if d['bias'] is None else d['bias'].cpu().numpy()
+        m = moe.MoELayer(d['router'].cpu().numpy(), d['gate_up'].reshape(-1), d['down'].reshape(-1), c['type'],
+                         c['experts'], c['hidden'], c['inter'], c['top_k'], router_b=bias)
+        return {'kind': kind, 'moe': m, 'h': d['h']}
+    cache = attention.KVCache(1, c['kv_heads'], c['head_dim'], _max_seq(c), c['heads'])
+    cache.k[0, :c['position'] + 1] = d['k']
+    cache.v[0, :c['position'] + 1] = d['v']
+    return {'kind': kind, 'cache': cache, 'q': d['q'], 'k': d['k_new'], 'v': d['v_new'], 'gate': d['gate'],
+            'position': c['position'], 'heads': c['heads'], 'window': c['window']}
+
+
+def run(s):
+    kind = s['kind']
+    if kind == 'matvec':
+        return s['q'].matvec(s['x'])
+    if kind == 'matmul':
+        return s['q'].matmul(s['x'])
+    if kind == 'chain':
+        return s['chain'].forward_device(s['pre'], s['att'], s['rope'])
+    if kind == 'moe':
+        return s['moe'].forward_device(s['h'])
+    cache = s['cache']
+    out = attention.attention_decode(s['q'], s['k'], s['v'], cache, 0, s['position'], s['heads'], window=s['window'],
+                                     gate=s['gate'])
+    return out, cache.k, cache.v
+
+
+# ---- what a pass cannot do without ---------------------------------------------
+
+def _matrix_bytes(t, values):
+    block, size = LAYOUT[t]
+    return values // block * size
+
+
+def _touched(c):
+    """Experts a MoE pass reads: the expected count of distinct experts of its tokens."""
+    e, k, n = c['experts'], c['top_k'], c['tokens']
+    if not c['zipf']:
+        return e * (1.0 - (1.0 - k / e) ** n)
+    # successive draws by popularity times a Gumbel-like spread: simulated once
+    r = np.random.default_rng(0)
+    p = np.arange(1, e + 1) ** -1.1
+    std = 0.02 * math.sqrt(c['hidden'])
+    logits = np.log(p / p.sum()) + std * r.standard_normal((n, e))
+    return len(np.unique(np.argsort(-logits, axis=1)[:, :k]))
+
+
+def work(case):
+    c = case
+    kind = c['kind']
+    if kind in ('matvec', 'matmul'):
+        r, k, n = c['rows'], c['cols'], c['tokens']
+        return {'bytes': _matrix_bytes(c['type'], r * k) + 4 * n * (r + k), 'flops': 2 * r * k * n}
+    if kind == 'chain':
+        shapes = _chain_shapes(c).values()
+        kv = c['kv_heads'] * c['head_dim']
+        vectors = 4 * (5 * c['dim'] + c['dim'] + 2 * kv + c['head_dim'])
+        return {'bytes': sum(_matrix_bytes(t, r * k) for t, r, k in shapes) + vectors,
+                'flops': sum(2 * r * k for _, r, k in shapes)}
+    if kind == 'moe':
+        n, e, h, i, k = c['tokens'], c['experts'], c['hidden'], c['inter'], c['top_k']
+        expert = _matrix_bytes(c['type'], 3 * h * i)
+        return {'bytes': 4 * e * h + _touched(c) * expert + 8 * n * h + 8 * n * k,
+                'flops': 2 * n * e * h + 6 * n * k * h * i}
+    n = c['position'] + 1
+    n = min(n, c['window']) if c['window'] else n
+    row = c['kv_heads'] * c['head_dim']
+    return {'bytes': 8 * row * n + 4 * (2 + int(c['gate'])) * c['heads'] * c['head_dim'] + 16 * row,
+            'flops': 4 * c['heads'] * c['head_dim'] * n}
+
+
+def tolerance(case):
+    kind = case['kind']
+    if kind == 'matvec':
+        # fp32-grade products (21 bits of x against its group's maximum)
+        return {'rel': 5e-6, 'max': 5e-5}
+    if kind == 'matmul' or (kind == 'moe' and case['tokens'] >= 32):
+        # f16 operands, fp32 sums: 2^-11 per product; expert choices follow fp64 sums
+        return {'rel': 1e-3, 'max': 1e-2, 'differ': 1e-3} if kind == 'moe' else {'rel': 1e-3, 'max': 1e-2}
+    if kind == 'moe':
+        return {'rel': 1e-5, 'max': 1e-4, 'differ': 1e-3}
+    if kind == 'chain':
+        # the matvecs' errors amplified by SiLU * up and two norms
+        return {'rel': 2e-5, 'max': 2e-4}
+    return {'rel': 2e-6, 'max': 2e-5}
+
+
+# ---- the same results in 64 bits -------------------------------------------------
+
+def _f16(b):
+    return b.contiguous().view(torch.float16).double()
+
+
+def _kq_scales(s):
+    """The eight 6-bit scales and minima of the 12-byte table s [blocks, 12]."""
+    s = s.to(torch.int32)
+    sc = torch.cat([s[:, :4] & 63, (s[:, 8:] & 15) | (s[:, :4] >> 6 << 4)], 1)
+    mn = torch.cat([s[:, 4:8] & 63, (s[:, 8:] >> 4) | (s[:, 4:8] >> 6 << 4)], 1)
+    return sc.double(), mn.double()
+
+
+def _decode(b, t):
+    """Values of GGML blocks b [blocks, bytes] in 64 bits, [blocks, values per block]."""
+    n = b.shape[0]
+    if t == 8:
+        return _f16(b[:, :2]) * b[:, 2:].contiguous().view(torch.int8).double()
+    if t == 2:
+        q = torch.cat([b[:, 2:] & 15, b[:, 2:] >> 4], 1)
+        return _f16(b[:, :2]) * (q.double() - 8.0)
+    if t in (12, 13):
+        d, dmin = _f16(b[:, :2]), _f16(b[:, 2:4])
+        sc, mn = _kq_scales(b[:, 4:16])
+        qs = b[:, 16 if t == 12 else 48:].reshape(n, 4, 32)
+        q = torch.stack([qs & 15, qs >> 4], 2).reshape(n, 8, 32)
+        if t == 13:
+            bit = torch.arange(8, device=b.device, dtype=torch.uint8).reshape(1, 8, 1)
+            q = q | ((b[:, 16:48].reshape(n, 1, 32) >> bit) & 1) << 4
+        return ((d * sc)[:, :, None] * q.double() - (dmin * mn)[:, :, None]).reshape(n, 256)
+    ql, qh = b[:, :128].reshape(n, 2, 64), b[:, 128:192].reshape(n, 2, 32)
+    lo = torch.stack([ql[:, :, :32] & 15, ql[:, :, 32:] & 15, ql[:, :, :32] >> 4, ql[:, :, 32:] >> 4], 2)
+    hi = torch.stack([qh & 3, qh >> 2 & 3, qh >> 4 & 3, qh >> 6], 2)
+    q = (lo | hi << 4).reshape(n, 16, 16).double() - 32.0
+    sc = b[:, 192:208].contiguous().view(torch.int8).double()
+    return ((_f16(b[:, 208:]) * sc)[:, :, None] * q).reshape(n, 256)
+
+
+def _product(raw, t, rows, cols, x):
+    """x [n, cols] (64 bits) times the transpose of the matrix in raw: [n, rows]."""
+    per = cols // LAYOUT[t][0]
+    step = max(1, (1 << 27) // cols)
+    out = []
+    for r in range(0, rows, step):
+        w = _decode(raw[r * per:min(rows, r + step) * per], t).reshape(-1, cols)
+        out.append(x @ w.T)
+    return torch.cat(out, 1)
+
+
+def _silu(x):
+    return x / (1.0 + torch.exp(-x))
+
+
+def _norm(x):
+    return x / torch.sqrt((x * x).mean() + EPS)
+
+
+def _rope(v, cos, sin, head_dim):
+    p = v.reshape(-1, head_dim // 2, 2)
+    a, b = p[..., 0], p[..., 1]
+    return torch.stack([a * cos - b * sin, a * sin + b * cos], -1).reshape(-1)
+
+
+def _exact_chain(c, d):
+    shapes = _chain_shapes(c)
+
+    def mul(n, v):
+        return _product(d['raws'][n], *shapes[n], v.reshape(1, -1)).reshape(-1)
+
+    x1 = d['pre'].double() + mul('attn_output', d['att'].double())
+    u = _norm(x1) * d['w_ffn'].double()
+    x = x1 + mul('ffn_down', _silu(mul('ffn_gate', u)) * mul('ffn_up', u))
+    v = _norm(x) * d['w_attn'].double()
+    cos, sin = d['cos'].double(), d['sin'].double()
+    return (x, _rope(mul('attn_q', v), cos, sin, c['head_dim']), _rope(mul('attn_k', v), cos, sin, c['head_dim']),
+            mul('attn_v', v))
+
+
+def _exact_moe(c, d):
+    h = d['h'].double()
+    logits = h @ d['router'].double().T
+    if d['bias'] is not None:
+        logits = logits + d['bias'].double()
+    logits = logits.float().double()
+    top, idx = torch.sort(logits, dim=1, descending=True, stable=True)
+    top, idx = top[:, :c['top_k']], idx[:, :c['top_k']]
+    gates = torch.softmax(top, 1)
+    e, hid, inter, t = c['experts'], c['hidden'], c['inter'], c['type']
+    gu = d['gate_up'].reshape(e, -1, LAYOUT[t][1])
+    dn = d['down'].reshape(e, -1, LAYOUT[t][1])
+    out = torch.zeros_like(h)
+    for x in torch.unique(idx).tolist():
+        tok, slot = torch.nonzero(idx == x, as_tuple=True)
+        y = _product(gu[x], t, 2 * inter, hid, h[tok])
+        y = _product(dn[x], t, hid, inter, _silu(y[:, :inter]) * y[:, inter:])
+        out.index_add_(0, tok, gates[tok, slot][:, None] * y)
+    return out, idx.to(torch.int32), gates
+
+
+def _exact_attention(c, d):
+    nh, nkv, hd, pos = c['heads'], c['kv_heads'], c['head_dim'], c['position']
+    cache = torch.zeros((2, 1, _max_seq(c), nkv, hd), dtype=torch.float32, device=_dev())
+    for i, (old, new) in enumerate(((d['k'], d['k_new']), (d['v'], d['v_new']))):
+        cache[i, 0, :pos + 1] = old
+        cache[i, 0, pos] = new.reshape(nkv, hd)
+    start = max(0, pos + 1 - c['window']) if c['window'] else 0
+    k, v = cache[0, 0, start:pos + 1].double(), cache[1, 0, start:pos + 1].double()
+    q = d['q'].double().reshape(nkv, nh // nkv, hd)
+    p = torch.softmax(torch.matmul(q, k.permute(1, 2, 0).contiguous()) / math.sqrt(hd), -1)
+    out = torch.matmul(p, v.permute(1, 0, 2).contiguous()).reshape(-1)
+    if d['gate'] is not None:
+        out = out / (1.0 + torch.exp(-d['gate'].double().clamp(-80.0, 80.0)))
+    return out, cache[0], cache[1]
+
+
+def exact(case, seed):
+    c, d = case, _inputs(case, seed)
+    if c['kind'] in ('matvec', 'matmul'):
+        y = _product(d['raw'], c['type'], c['rows'], c['cols'], d['x'].double())
+        return y.reshape(-1) if c['kind'] == 'matvec' and c['tokens'] == 1 else y
+    if c['kind'] == 'chain':
+        return _exact_chain(c, d)
+    if c['kind'] == 'moe':
+        return _exact_moe(c, d)
+    return _exact_attention(c, d)
