@@ -49,14 +49,14 @@ def _compile(src: Path) -> Path:
 # LDS stages filled by global_load_lds, n copies per stage and wave (n = 0: a
 # double buffer, whose every copy from before the last barrier has landed by
 # the LDS reads after it)
-COUNTED_LOADS = [('gemm.hip', 'gemm_cu_q80_kernel', None), ('moe.hip', 'moe_route_logits_kernel', 4),
-                 ('gemm.hip', 'gemm_tile_kernel', 0)]
+COUNTED_LOADS = [('moe.hip', 'moe_route_logits_kernel', 4), ('gemm.hip', 'gemm_tile_kernel', 0),
+                 ('gemm_dense.hip', 'gemm_dense_kernel', None), ('gemm_dense.hip', 'gemm_dense_kernel', 4)]
 
 
 def _check(item) -> None:
     from .isa_check import check_lds_ring, check_source
     src, kernel, per_stage = item
-    out = BUILD / (src + '.' + kernel + '.s')
+    out = BUILD / f'{src}.{kernel}.{per_stage}.s'
     if per_stage is None:
         check_source(HIPCC, COMMON, CSRC / src, kernel, out)
     else:

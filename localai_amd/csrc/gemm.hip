@@ -10,36 +10,27 @@
 // by a power of two so that its largest magnitude lies in [2^14, 2^15)
 // (exact), rounded to f16, and the output is scaled back by the inverse power.
 // f16 (11 significant bits) rather than bf16 (8) keeps the normwise error near
-// 2^-12. The rows are stored row-major, or (for the CU-tile kernel) in MFMA
-// operand order, 1 KB per 16 tokens x 32 values.
+// 2^-12.
 //
 // Three kernels:
-//   gemm_kernel       any type from the GGML bytes: a workgroup decodes a
-//                     128-row weight tile into LDS per 128-value step and 4
-//                     waves multiply it with 128 tokens (also the MoE expert
-//                     tiles of moe.hip);
-//   gemm_tile_kernel  Q4_K / Q6_K / Q8_0 from the tile form (mfma_core.h):
-//                     each wave decodes its own two 16-row tiles into B
-//                     operands in registers, x is staged in LDS
-//                     (global_load_lds), dense and MoE;
-//   gemm_cu_q80_kernel dense Q8_0 with 256 tokens or more: one 224-row x
-//                     128-token tile per CU, sized to what L2 can feed a CU
-//                     (its own section below).
+//   gemm_dense_kernel (gemm_dense.hip) every dense product on the tile form
+//                     (Q4_K / Q6_K / Q8_0);
+//   gemm_tile_kernel  the MoE expert tiles on the tile form: each wave decodes
+//                     its own two 16-row tiles into B operands in registers, x
+//                     is staged in LDS (global_load_lds);
+//   gemm_kernel       types without a tile form (Q4_0, Q5_K), dense and expert
+//                     tiles, from the row planes: a workgroup decodes a 128-row
+//                     weight tile into LDS per 128-value step and 4 waves
+//                     multiply it with 128 tokens.
 #include <type_traits>
 
-#include "f16rows.h"
-#include "gemv_core.h"
-#include "internal.h"
-#include "mfma_core.h"
+#include "gemm_core.h"
 
 namespace lq {
-
-typedef _Float16 lq_h8 __attribute__((ext_vector_type(8)));
 
 constexpr int GM_BM = 128;             // weight rows per workgroup
 constexpr int GM_BN = 128;             // tokens per workgroup (dense)
 constexpr int GM_MOE_BN = 64;          // tokens per workgroup (MoE expert tiles)
-constexpr int GM_BK = 128;             // K values per step (two 64-value units)
 constexpr int GM_LD = GM_BK + 8;       // LDS row stride in halves (272 B: 16 lanes of a
                                        // 16-byte read hit 16 distinct bank groups)
 
@@ -50,10 +41,9 @@ template <int NG>
 __global__ __launch_bounds__(256) void x_to_f16_kernel(const float *__restrict__ X, int64_t ldx, int cols,
                                                        const int32_t *__restrict__ rows_map, int k, int64_t ntok,
                                                        _Float16 *__restrict__ Xh, int ldh,
-                                                       float *__restrict__ inv, int vec, int tiled, int64_t ntok_pad,
-                                                       float *__restrict__ nrm2) {
+                                                       float *__restrict__ inv, int vec, float *__restrict__ nrm2) {
     const int64_t t = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_id();
-    x_to_f16_row<NG>(t, X, ldx, cols, rows_map, k, ntok, Xh, ldh, inv, vec, tiled, ntok_pad, nrm2);
+    x_to_f16_row<NG>(t, X, ldx, cols, rows_map, k, ntok, Xh, ldh, inv, vec, nrm2);
 }
 
 // ---------------------------------------------------------------- weights
@@ -123,72 +113,12 @@ __device__ __forceinline__ int window_pos(int u, int j) {
     else return 64 * (u & 1) + j;
 }
 
-typedef _Float16 lq_h2 __attribute__((ext_vector_type(2)));
-
-// Bytes 0, 1 (lo) or 2, 3 (hi) of w below the exponent byte 0x64: two f16
-// values 1024 + byte (one v_perm_b32; selector bytes 0..3 pick w's bytes,
-// 4 picks the first byte of 0x64646464).
-__device__ __forceinline__ uint32_t f16_bytes_lo(uint32_t w) {
-    return __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u);
-}
-__device__ __forceinline__ uint32_t f16_bytes_hi(uint32_t w) {
-    return __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u);
-}
-
-// Q8_0 weights straight to f16 pairs: byte q + 128 under the f16 exponent of
-// 1024 reads as 1152 + q (exact), minus 1152 gives q exactly, and one f16
-// multiply by d rounds d * q once (the same value as rounding the exact fp32
-// product). Four int8 quants in `w` -> two f16 pairs.
-__device__ __forceinline__ void q8_pairs(uint32_t w, lq_h2 d2, uint32_t &lo, uint32_t &hi) {
-    const uint32_t b = w ^ 0x80808080u;
-    const uint32_t l = f16_bytes_lo(b), h = f16_bytes_hi(b);
-    const lq_h2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    lo = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(lq_h2, l) - off) * d2);
-    hi = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(lq_h2, h) - off) * d2);
-}
-
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     const _Float16 ha = (_Float16)a, hb = (_Float16)b;
     return (uint32_t)__builtin_bit_cast(uint16_t, ha) | ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
 }
 
 // ---------------------------------------------------------------- GEMM
-
-enum { GM_DENSE = 0, GM_MOE_GATE_UP = 1, GM_MOE_DOWN = 2 };
-
-// Dense: token tile blockIdx.y of Xh [ntok, ldh]; Y[t * y_ts + r * y_rs].
-// MoE: work tile blockIdx.y of the expert tile list (expert, first row of
-// the expert-major Xh, valid rows); gate_up writes silu(g) * u to
-// Y[p * y_ts + r] for r < inter, down writes Y[p * y_ts + r].
-struct GemmArgs {
-    lq_geom g;
-    const uint8_t *W;          // dense: the matrix; MoE: expert 0 of the [E, rows, cols] handle
-    const _Float16 *Xh;        // f16 rows, stride ldh (zero past cols)
-    int ldh;
-    const float *inv;          // per Xh row output scale
-    int64_t ntok;
-    float *Y;
-    int64_t y_ts, y_rs;
-    const int32_t *tile_e, *tile_p0, *tile_n, *n_tiles;
-    int64_t inter;
-    const uint8_t *Wt;         // tile form (mfma_core.h) or null; MoE: expert 0
-    int64_t wt_bytes;          // tile-form bytes per matrix
-    const int32_t *rows_map;   // null, or: token p reads Xh / inv row rows_map[p] / rows_k
-    int rows_k;
-    // MoE gate_up on the tile form, f16 output (Yh not null): SiLU * up of
-    // token p goes to Yh row p (stride ldy) times 2^s, inv_out[p] = 2^-s, s
-    // from the bound 4 |gate rows| |up rows| |h row|^2 (wnorm: the expert
-    // handle's row_norm, xnorm2: sum of squares per Xh row)
-    _Float16 *Yh;
-    int64_t ldy;
-    float *inv_out;
-    const float *wnorm, *xnorm2;
-};
-
-// Xh / inv row of token position p
-__device__ __forceinline__ int64_t gemm_xrow(const GemmArgs &a, int64_t p) {
-    return a.rows_map ? (int64_t)(a.rows_map[p] / a.rows_k) : p;
-}
 
 template <int T, int BN, int MODE>
 __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
@@ -362,37 +292,12 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 // weight rows straight into B registers -- each weight value once per
 // workgroup, exactly in fp32 (or, for Q8_0, exactly as 1152 + q in f16 times
 // d), rounded once to f16 -- and only the f16 activations (A operands) go
-// through LDS, double-buffered and shared by the 4 waves.
+// through LDS, double-buffered and shared by the waves.
 //
-// Workgroup: 4 waves x 2 row tiles (128 weight rows; for gate_up 64 gate rows
-// and the 64 matching up rows) x BN tokens, 128 K values per step.
+// Workgroup: 8 waves x 2 row tiles (256 weight rows; for gate_up 128 gate rows
+// and the 128 matching up rows) x 64 tokens, 128 K values per step.
 
-// Workgroup barrier without the fence of __syncthreads, whose wait for every
-// outstanding LDS read would stall on the next step's operand prefetch. What
-// crosses it is ordered by hand: each wave waits (vmcnt) for its own copies
-// into the ring before arriving, and every read of a ring slot has been
-// consumed by an MFMA (lgkmcnt wait) before the barrier that precedes the
-// slot's refill. The memory clobber keeps the compiler from moving memory
-// accesses across it.
-__device__ __forceinline__ void cu_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-// 1 KB from global memory (16 bytes per lane) into LDS at the wave-uniform
-// byte address lds (lane i's bytes at lds + 16 i), through M0, which it saves
-// and restores
-__device__ __forceinline__ void cu_dma(const void *src, uint32_t lds) {
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep)
-                 : "v"(src), "s"(lds)
-                 : "memory");
-}
-constexpr int GT_WROWS = 128;          // weight rows per workgroup (dense, 4 waves)
 constexpr int GM_MOE_NW = 8;           // waves per workgroup of the expert tile GEMMs
-
-template <int T> struct GtRaw;
-template <> struct GtRaw<LQ_Q4_K> { uint4 qs, hd; };
-template <> struct GtRaw<LQ_Q6_K> { uint4 ql, qh, sc; uint32_t d; };
-template <> struct GtRaw<LQ_Q8_0> { uint4 p0, p1, dd; };
 
 // weights of half `half` (values 128 half .. + 127) of one 256-value block
 template <int T>
@@ -417,95 +322,13 @@ __device__ __forceinline__ GtRaw<T> gt_load(const uint8_t *blk, int half, int la
     return r;
 }
 
-// Q4_K sub-block scale pair {d * sc, dmin * mn} (packed f16, each rounded
-// once) of row lane % 16, sub-block 4 HALF + lane / 16: the four lane groups
-// of a wave cover the four sub-blocks of a half at once; gt_b fetches the
-// pair of its own sub-block from the lane that computed it
-template <int HALF>
-__device__ __forceinline__ uint32_t gt_q4k_pair(const uint4 &hd, int q) {
-    const uint32_t s0 = hd.y, s4 = hd.z, s8 = hd.w;   // scale bytes 0..3, 4..7, 8..11
-    uint32_t sc, mn;
-    if constexpr (HALF == 0) {
-        sc = __builtin_amdgcn_ubfe(s0, 8 * q, 6);
-        mn = __builtin_amdgcn_ubfe(s4, 8 * q, 6);
-    } else {
-        sc = __builtin_amdgcn_ubfe(s8, 8 * q, 4) | (__builtin_amdgcn_ubfe(s0, 8 * q + 6, 2) << 4);
-        mn = __builtin_amdgcn_ubfe(s8, 8 * q + 4, 4) | (__builtin_amdgcn_ubfe(s4, 8 * q + 6, 2) << 4);
-    }
-    // packed f16: {sc, mn} exactly (0x6400 | n reads as 1024 + n), times
-    // {d, dmin} rounds d * sc and dmin * mn once each
-    const lq_h2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-    const lq_h2 scmn = __builtin_bit_cast(lq_h2, sc | (mn << 16) | 0x64006400u) - k1024;
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(lq_h2, hd.x) * scmn);
-}
-
-// B operand (8 f16) of slice kk (0..3) of half HALF of the block, lane group
-// q; Q4_K: pair = the slice's scale pair for the lane's row (gt_q4k_pair)
-template <int T, int HALF, int KK>
-__device__ __forceinline__ lq_h8 gt_b(const GtRaw<T> &r, int q, uint32_t pair_ab = 0) {
-    uint4 o;
-    if constexpr (T == LQ_Q4_K) {
-        // group g = 4 HALF + KK: qs chunk g / 2 (bytes 8 ((g / 2) % 2) ..), nibble g % 2;
-        // a value is round(a * q - b) from the exact q (one fused multiply-add)
-        constexpr int g = 4 * HALF + KK, hb = (g >> 1) & 1, nib = g & 1;
-        const lq_h2 ab = __builtin_bit_cast(lq_h2, pair_ab);
-        const lq_h2 a2 = {ab.x, ab.x}, nb2 = {-ab.y, -ab.y};
-        const uint32_t w0 = ((hb ? r.qs.z : r.qs.x) >> (4 * nib)) & 0x0F0F0F0Fu;
-        const uint32_t w1 = ((hb ? r.qs.w : r.qs.y) >> (4 * nib)) & 0x0F0F0F0Fu;
-        // the byte 0000qqqq read as FP8 e4m3 is exactly q 2^-9 (subnormal
-        // below 8, normal from 8 on); the scaled conversion times 2^9 gives
-        // two f16 q exactly in one instruction
-        auto fma2 = [&](lq_h2 q) { return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, a2, nb2)); };
-        o.x = fma2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 512.0f, false));
-        o.y = fma2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 512.0f, true));
-        o.z = fma2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 512.0f, false));
-        o.w = fma2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 512.0f, true));
-    } else if constexpr (T == LQ_Q6_K) {
-        // slice g = 4 HALF + KK: values 128 HALF + 32 KK + 8q .. ; ql nibble KK / 2 of
-        // bytes 8 (KK % 2) ..; qh bits 2 KK of bytes 8 HALF ..; sub-block 2g + q / 2
-        constexpr int g = 4 * HALF + KK;
-        const uint32_t l0 = ((KK & 1) ? r.ql.z : r.ql.x) >> (4 * (KK >> 1));
-        const uint32_t l1 = ((KK & 1) ? r.ql.w : r.ql.y) >> (4 * (KK >> 1));
-        const uint32_t e0 = (HALF ? r.qh.z : r.qh.x) >> (2 * KK), e1 = (HALF ? r.qh.w : r.qh.y) >> (2 * KK);
-        const uint32_t w0 = (l0 & 0x0F0F0F0Fu) | ((e0 & 0x03030303u) << 4);
-        const uint32_t w1 = (l1 & 0x0F0F0F0Fu) | ((e1 & 0x03030303u) << 4);
-        // sub-blocks 2g and 2g + 1 share scale dword g / 2
-        const uint32_t sw = (g >> 1) == 0 ? r.sc.x : (g >> 1) == 1 ? r.sc.y : (g >> 1) == 2 ? r.sc.z : r.sc.w;
-        const int sbyte = ((2 * g) & 3) + (q >> 1);
-        // packed f16: 1024 + q minus 1056 is q - 32 exactly; times d * sc
-        // (rounded once) rounds each value once
-        const _Float16 dsc = __builtin_bit_cast(_Float16, (uint16_t)(r.d & 0xFFFFu)) *
-                             (_Float16)(int)__builtin_amdgcn_sbfe((int)sw, 8 * sbyte, 8);
-        const lq_h2 d2 = {dsc, dsc}, k1056 = {(_Float16)1056.0f, (_Float16)1056.0f};
-        auto pair = [&](uint32_t bits) {
-            return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(lq_h2, bits) - k1056) * d2);
-        };
-        o.x = pair(f16_bytes_lo(w0));
-        o.y = pair(f16_bytes_hi(w0));
-        o.z = pair(f16_bytes_lo(w1));
-        o.w = pair(f16_bytes_hi(w1));
-    } else {
-        // GGML block 4 HALF + KK: piece KK / 2 of the half, bytes 8 (KK % 2) ..
-        const uint4 pc = (KK >> 1) ? r.p1 : r.p0;
-        const uint32_t w0 = (KK & 1) ? pc.z : pc.x, w1 = (KK & 1) ? pc.w : pc.y;
-        constexpr int g = 4 * HALF + KK;
-        const uint32_t dw = g < 2 ? r.dd.x : g < 4 ? r.dd.y : g < 6 ? r.dd.z : r.dd.w;
-        const uint32_t dh = (dw >> (16 * (g & 1))) & 0xFFFFu;
-        const lq_h2 d2 = __builtin_bit_cast(lq_h2, dh * 0x10001u);
-        q8_pairs(w0, d2, o.x, o.y);
-        q8_pairs(w1, d2, o.z, o.w);
-    }
-    return __builtin_bit_cast(lq_h8, o);
-}
-
 // MFMAs of the four 32-value slices of half HALF of a block: B operands
 // decoded from the wave's two row tiles, A operands from the LDS x tile
 // x tile in LDS: [token][16 chunks of 8 halves], chunk c of token t stored at
 // position c ^ (t % 16), so the 16 tokens of an A read hit 16 bank groups.
 // The wave raises its priority while it issues a slice's MFMAs, so the wave
 // that holds ready MFMAs keeps the matrix core of its SIMD (the waves of a
-// SIMD come from different workgroups). Dense 14336 x 4096 x 512 Q8_0: 88 us
-// against 97 us; the expert GEMMs gain about 1 %.
+// SIMD come from different workgroups); the expert GEMMs gain about 1 %.
 // Q4_K: pr0 / pr1 are the scale pairs of this half (gt_q4k_pair), computed
 // by the caller while half 0's scale registers are live
 template <int T, int HALF, int NI>
@@ -753,33 +576,16 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) 
     // wave index made wave-uniform: row-tile addresses go to scalar registers
     // (MoE Q4_K GEMMs 162 -> 128 VGPRs; gate_up 85 -> 81 us, down 55 -> 48 us)
     const int wave = wave_id();
-    const uint8_t *Wt = a.Wt;
-    int64_t p0;
-    int tn;
-    int64_t blk;
-    const float *wn = nullptr;   // the expert's row norms (gate_up with f16 output)
-    if constexpr (MODE == GM_DENSE) {
-        // 1-D grid, padded to a multiple of 8; workgroup id -> logical index
-        // xcd * per + id / 8 walks the row blocks of one token tile per XCD
-        const int id = blockIdx.x, per = gridDim.x / 8;
-        const int L = (id % 8) * per + id / 8;
-        const int nrb = (int)((g.rows + 32 * NW - 1) / (32 * NW));
-        const int64_t ntt = (a.ntok + BN - 1) / BN;
-        if (L >= nrb * ntt) return;
-        blk = L % nrb;
-        p0 = (int64_t)(L / nrb) * BN;
-        tn = (int)(a.ntok - p0 < BN ? a.ntok - p0 : BN);
-    } else {
-        blk = blockIdx.x;
-        const int tile = blockIdx.y;
-        if (tile >= a.n_tiles[0]) return;
-        Wt += (int64_t)a.tile_e[tile] * a.wt_bytes;
-        if (a.wnorm) wn = a.wnorm + 2 * (int64_t)a.tile_e[tile];
-        p0 = a.tile_p0[tile];
-        tn = a.tile_n[tile];
-    }
+    const int64_t blk = blockIdx.x;
+    const int tile = blockIdx.y;
+    if (tile >= a.n_tiles[0]) return;
+    const uint8_t *Wt = a.Wt + (int64_t)a.tile_e[tile] * a.wt_bytes;
+    // the expert's row norms (gate_up with f16 output)
+    const float *wn = a.wnorm ? a.wnorm + 2 * (int64_t)a.tile_e[tile] : nullptr;
+    const int64_t p0 = a.tile_p0[tile];
+    const int tn = a.tile_n[tile];
     const int64_t tiles = (g.rows + MT_ROWS - 1) / MT_ROWS, nsb = mt_nsb(g);
-    // the wave's two row tiles: dense / down 2 NW blk + 2 wave + j; gate_up
+    // the wave's two row tiles: down 2 NW blk + 2 wave + j; gate_up
     // gate tile NW blk + wave (j = 0) and its up tile inter / 16 + NW blk + wave
     int64_t t0, t1;
     if constexpr (MODE == GM_MOE_GATE_UP) {
@@ -791,291 +597,13 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) 
     }
     const uint8_t *w0p = Wt + (t0 < tiles ? t0 : tiles - 1) * nsb * BB;
     const uint8_t *w1p = Wt + (t1 < tiles ? t1 : tiles - 1) * nsb * BB;
-    if constexpr (MODE == GM_DENSE || NI != 4) {
-        gt_main<T, BN, MODE, NW, NI>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-    } else {
-        // expert tiles: one copy of the loop per count of 16-token tiles
-        const int nv = __builtin_amdgcn_readfirstlane((tn + 15) >> 4);
-        if (nv == 1) gt_main<T, BN, MODE, NW, 1>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-        else if (nv == 2) gt_main<T, BN, MODE, NW, 2>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-        else if (nv == 3) gt_main<T, BN, MODE, NW, 3>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-        else gt_main<T, BN, MODE, NW, 4>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-    }
-}
-
-// ---------------------------------------------------------------- CU-tile GEMM (Q8_0, many tokens)
-
-// One workgroup per CU owns a 224-row x 128-token output tile (14 row tiles
-// x 8 token tiles; 14336 x 512 is exactly 256 such tiles). The shape follows
-// from what a CU can be fed: L2 delivers about 32 B per clock to a CU (1 KB
-// contiguous per load instruction; half that for 64-byte pieces of rows 8 KB
-// apart). Per 64-value K step the tile needs 128 tokens x 128 B of x and 224
-// rows x 68 B of Q8_0 weights, about 31 KB, roughly what L2 delivers in the
-// time of the step's MFMAs.
-//
-// Waves 0..6 compute: wave w owns row tiles 2w, 2w + 1 for all 8 token tiles
-// (32 v_mfma_f32_16x16x32_f16 per step). It loads its own raw weights (tile
-// form, 1 KB contiguous per load) and decodes them in registers straight into
-// MFMA A operands, so weights never pass through LDS. x (the tiled form of
-// x_to_f16, 16 KB per step: 8 token tiles x 2 slices, 1 KB each in lane
-// order) goes into a 4-step LDS ring three steps ahead, wave w copying token
-// tile w with global_load_lds; the compute waves read it as B operands (one
-// conflict-free ds_read_b128 per token tile and slice). With the weights as
-// A and the tokens as B, each lane ends up holding 4 consecutive rows of one
-// token, stored as one 16-byte write. Ring slot (j + 3) % 4 is refilled at
-// step j, after the barrier that ended step j - 1, its last reader. One
-// workgroup barrier per step.
-//
-// The compute waves' weight loads are asm whose completion the kernel counts
-// itself (4 loads per step); every use goes through cu_wait_w, which
-// names the registers, and the build checks the generated code for any
-// instruction touching a register whose load may still be in flight. The
-// MFMAs are asm with the accumulators in VGPRs: as builtins, the register
-// allocator rotated the accumulators through copies at every iteration of
-// the unrolled loop, and in AGPRs the compiler capped the VGPRs at 128 and
-// spilled (copied) registers with loads in flight into AGPRs.
-constexpr int CU_RT = 14;                        // row tiles per workgroup
-constexpr int CU_TT = 8;                         // token tiles per workgroup
-constexpr int CU_WR = 2;                         // row tiles per compute wave
-constexpr int CU_NC = 7;                         // compute waves
-constexpr int CU_RING = 4;                       // x ring depth (steps)
-constexpr int CU_XSTEP = CU_TT * 2 * 1024;       // x bytes per step
-constexpr int CU_TOKENS = CU_TT * 16;
-// LDS requested per workgroup: more than half of a CU's 160 KB (the ring uses
-// 64 KB), so that no CU holds two workgroups (a second one would halve that
-// CU's MFMA rate and leave another CU idle)
-constexpr int CU_LDS_RESERVE = 96 * 1024;
-static_assert(CU_RING * CU_XSTEP <= CU_LDS_RESERVE, "CU-tile LDS");
-
-// global loads with a wave-uniform 64-bit base in SGPRs and a 32-bit per-lane
-// byte offset (fewer VGPRs than 64-bit addresses per load)
-__device__ __forceinline__ void cu_load(mt_i4 &v, const void *base, uint32_t off) {
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(off), "s"(base) : "memory");
-}
-__device__ __forceinline__ void cu_load(int &v, const void *base, uint32_t off) {
-    asm volatile("global_load_dword %0, %1, %2" : "=v"(v) : "v"(off), "s"(base) : "memory");
-}
-template <int N, class W>
-__device__ __forceinline__ void cu_wait_w(W &w) {
-    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0].q), "+v"(w[0].d), "+v"(w[1].q), "+v"(w[1].d) : "n"(N) : "memory");
-}
-
-// XCD-aware tile order. Workgroups go to the 8 XCDs round robin
-// (blockIdx.x % 8); renumbered, each XCD runs a contiguous range, ordered as
-// groups of (up to) 4 token blocks of one row block. The 4 workgroups of a
-// row block then run side by side on one XCD and read each weight step from
-// its L2 (HBM reads the 62 MB of 14336 x 4096 weights once), and the XCD's
-// workgroups, all at similar K positions, share the x steps in L2 as well.
-__device__ __forceinline__ void cu_tile(int nrb, int ntb, int &rb, int &tb) {
-    const int G = gridDim.x, per = G / 8, rem = G % 8, xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
-    const int L = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-    const int tq = L / (4 * nrb), r = L % (4 * nrb), gs = ntb - 4 * tq < 4 ? ntb - 4 * tq : 4;
-    rb = r / gs;
-    tb = 4 * tq + r % gs;
-}
-
-// y_vec: Y rows are contiguous (y_rs 1), 16-byte aligned, y_ts % 4 == 0
-__global__ __launch_bounds__(512, 1) void gemm_cu_q80_kernel(GemmArgs a, int nrb, int ntb, int y_vec) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t cu_lds[];
-    const lq_geom &g = a.g;
-    const int lane = lane_id(), w = wave_id();
-    int rb, tb;
-    cu_tile(nrb, ntb, rb, tb);
-    const int64_t tiles = (g.rows + MT_ROWS - 1) / MT_ROWS, nsb = mt_nsb(g);
-    const int64_t p0 = (int64_t)tb * CU_TOKENS, t0 = (int64_t)rb * CU_RT;
-    const int nsteps = (int)(nsb * 4);               // 64-value steps (a multiple of 4)
-
-    // x: wave w copies token tile w (both 32-value slices, 2 KB) of each step
-    // into the ring; the compute waves read every token tile
-    const int64_t nks = a.ldh / 32, ttiles = (a.ntok + 15) / 16;
-    int64_t xtt = p0 / 16 + w;
-    xtt = xtt < ttiles ? xtt : ttiles - 1;
-    const uint8_t *const xsrc = reinterpret_cast<const uint8_t *>(a.Xh) + xtt * nks * 1024 + 16 * lane;
-    const uint32_t ring = (uint32_t)(uintptr_t)cu_lds + 2048 * w;
-    auto dma = [&](int j) {                          // 2 loads
-        const int jj = j < nsteps ? j : nsteps - 1;
-        const uint32_t dst = ring + (j % CU_RING) * CU_XSTEP;
-        cu_dma(xsrc + 2048 * jj, dst);
-        cu_dma(xsrc + 2048 * jj + 1024, dst + 1024);
-    };
-    dma(0);
-    dma(1);
-    dma(2);
-
-    if (w == CU_NC) {
-        // ---- the eighth wave only copies: x(j + 1) (requested at step j - 2)
-        // is complete once at most the 4 loads of steps j - 1 and j are in flight
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        for (int j = 0; j < nsteps; ++j) {
-            dma(j + 3);
-            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-            cu_barrier();
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        return;
-    }
-
-    // ---- compute waves
-    uint32_t woff[CU_WR];
-#pragma unroll
-    for (int r = 0; r < CU_WR; ++r) {
-        int64_t t = t0 + CU_WR * w + r;
-        t = t < tiles ? t : tiles - 1;
-        woff[r] = (uint32_t)(t * nsb * MT_Q80_BLOCK);
-    }
-    const uint32_t qlane = 16 * lane, dlane = 4096 + 16 * (lane & 15);
-    struct WRaw { mt_i4 q; int d; };
-    auto load_w = [&](WRaw (&dst)[CU_WR], int j) {    // 4 loads
-        j = j < nsteps ? j : nsteps - 1;
-        const int blk = j >> 2, piece = j & 3;
-        const uint8_t *qb = a.Wt + (int64_t)blk * MT_Q80_BLOCK + piece * 1024, *db = a.Wt + (int64_t)blk * MT_Q80_BLOCK + 4 * piece;
-#pragma unroll
-        for (int r = 0; r < CU_WR; ++r) {
-            cu_load(dst[r].q, qb, woff[r] + qlane);
-            cu_load(dst[r].d, db, woff[r] + dlane);
-        }
-    };
-    typedef lq_h8 WOps[CU_WR][2];
-    auto decode = [&](WRaw (&src)[CU_WR], WOps &o) {
-#pragma unroll
-        for (int r = 0; r < CU_WR; ++r) {
-            const uint32_t d = (uint32_t)src[r].d;
-            const lq_h2 d0 = __builtin_bit_cast(lq_h2, (d & 0xFFFFu) * 0x10001u);
-            const lq_h2 d1 = __builtin_bit_cast(lq_h2, (d >> 16) * 0x10001u);
-            uint4 o0, o1;
-            q8_pairs((uint32_t)src[r].q[0], d0, o0.x, o0.y);
-            q8_pairs((uint32_t)src[r].q[1], d0, o0.z, o0.w);
-            q8_pairs((uint32_t)src[r].q[2], d1, o1.x, o1.y);
-            q8_pairs((uint32_t)src[r].q[3], d1, o1.z, o1.w);
-            o[r][0] = __builtin_bit_cast(lq_h8, o0);
-            o[r][1] = __builtin_bit_cast(lq_h8, o1);
-        }
-    };
-
-    lq_f4 acc[CU_WR][CU_TT];
-#pragma unroll
-    for (int r = 0; r < CU_WR; ++r)
-#pragma unroll
-        for (int i = 0; i < CU_TT; ++i) acc[r][i] = lq_f4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // x B operands: slice sl of step j is read into xv[sl] as soon as the
-    // MFMAs of slice sl of step j - 1 are issued (x(j) has been in LDS since
-    // the barrier that ended step j - 2), so the reads overlap MFMAs
-    typedef lq_h8 XOps[2][CU_TT];
-    auto read_x = [&](int j, XOps &xv, int sl) {
-        const uint8_t *xs = cu_lds + (j % CU_RING) * CU_XSTEP + 16 * lane + sl * 1024;
-#pragma unroll
-        for (int i = 0; i < CU_TT; ++i) xv[sl][i] = *reinterpret_cast<const lq_h8 *>(xs + 2048 * i);
-    };
-    auto mfmas = [&](int j, XOps &xv, WOps &cur) {
-#pragma unroll
-        for (int sl = 0; sl < 2; ++sl) {
-#pragma unroll
-            for (int i = 0; i < CU_TT; ++i)
-#pragma unroll
-                for (int r = 0; r < CU_WR; ++r)
-                    asm("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[r][i]) : "v"(cur[r][sl]), "v"(xv[sl][i]));
-            read_x(j + 1, xv, sl);
-        }
-    };
-
-    // Raw weights run 4 steps ahead in 4 register sets. Each step a compute
-    // wave requests its 2 KB of x(j + 3), then 4 weight loads: the raw set
-    // decoded at step j was requested at step j - 4 and is complete once at
-    // most the 18 loads of steps j - 3 .. j - 1 are in flight; the wave's own
-    // part of x(j + 1), requested at step j - 2, once at most 16 are (the
-    // weights of step j - 2 and steps j - 1, j), and the barrier then makes
-    // all of x(j + 1) visible. One decoded operand set: the MFMAs read their
-    // operands at issue, so the decode may overwrite them once the step's
-    // MFMAs are issued. The two compute waves of a SIMD (w and w + 4) run
-    // opposite phases, one issuing MFMAs while the other decodes:
-    //   waves 0..3, step j: MFMAs(j); decode W(j + 1); request x(j + 3), W(j + 5)
-    //   waves 4..6, step j: decode W(j); request x(j + 3), W(j + 4); MFMAs(j)
-    // Everything the prologue requested has landed before the loop: the
-    // compiler may copy loop-carried registers on entry, and a copy of a
-    // register still waiting for its load would read stale data.
-    WRaw wr[4][CU_WR];
-    WOps cur;
-    XOps xv;
-    if (w < 4) {
-        WRaw w0[CU_WR];
-        load_w(w0, 0);
-#pragma unroll
-        for (int k = 1; k <= 4; ++k) load_w(wr[k & 3], k);
-        cu_wait_w<16>(w0);
-        decode(w0, cur);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cu_wait_w<0>(wr[k]);
-        __syncthreads();
-        read_x(0, xv, 0);
-        read_x(0, xv, 1);
-        auto step = [&](int j, WRaw (&w1)[CU_WR]) {
-            mfmas(j, xv, cur);
-            cu_wait_w<18>(w1);
-            decode(w1, cur);                    // past the end: a clamped copy nobody uses
-            dma(j + 3);
-            load_w(w1, j + 5);
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // own part of x(j + 1)
-            cu_barrier();
-        };
-        for (int j = 0; j < nsteps; j += 4) {
-            step(j, wr[1]);
-            step(j + 1, wr[2]);
-            step(j + 2, wr[3]);
-            step(j + 3, wr[0]);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) load_w(wr[k], k);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cu_wait_w<0>(wr[k]);
-        __syncthreads();
-        read_x(0, xv, 0);
-        read_x(0, xv, 1);
-        auto step = [&](int j, WRaw (&w0)[CU_WR]) {
-            cu_wait_w<18>(w0);
-            decode(w0, cur);
-            dma(j + 3);
-            load_w(w0, j + 4);
-            mfmas(j, xv, cur);
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // own part of x(j + 1)
-            cu_barrier();
-        };
-        for (int j = 0; j < nsteps; j += 4) {
-            step(j, wr[0]);
-            step(j + 1, wr[1]);
-            step(j + 2, wr[2]);
-            step(j + 3, wr[3]);
-        }
-    }
-    // the loads past the end land in registers the compiler counts as free;
-    // and the MFMAs are asm, so the compiler does not know to wait for their
-    // results before reading the accumulators: 24 wait states cover the
-    // longest (16-pass) MFMA write-to-read distance
-    asm volatile("s_waitcnt vmcnt(0)\n s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
-
-    // D: lane holds rows 4 (lane / 16) + v of a row tile, token lane % 16 of a token tile
-#pragma unroll
-    for (int i = 0; i < CU_TT; ++i) {
-        const int64_t p = p0 + 16 * i + (lane & 15);
-        if (p >= a.ntok) continue;
-        const float sc = a.inv[p];
-        float *yp = a.Y + p * a.y_ts;
-#pragma unroll
-        for (int r = 0; r < CU_WR; ++r) {
-            const int64_t t = t0 + CU_WR * w + r, row = t * MT_ROWS + 4 * (lane >> 4);
-            if (t >= tiles) continue;
-            const lq_f4 v = acc[r][i] * sc;
-            if (y_vec && row + 3 < g.rows) {
-                *reinterpret_cast<lq_f4 *>(yp + row) = v;
-            } else {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (row + k < g.rows) yp[(row + k) * a.y_rs] = v[k];
-            }
-        }
-    }
+    // one copy of the loop per count of 16-token tiles
+    static_assert(BN == 64, "up to four 16-token tiles");
+    const int nv = __builtin_amdgcn_readfirstlane((tn + 15) >> 4);
+    if (nv == 1) gt_main<T, BN, MODE, NW, 1>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    else if (nv == 2) gt_main<T, BN, MODE, NW, 2>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    else if (nv == 3) gt_main<T, BN, MODE, NW, 3>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    else gt_main<T, BN, MODE, NW, 4>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
 }
 
 // ---------------------------------------------------------------- host side
@@ -1084,127 +612,31 @@ __global__ __launch_bounds__(512, 1) void gemm_cu_q80_kernel(GemmArgs a, int nrb
 // tile form's block; a multiple of the row-plane kernel's 128-value step)
 static int64_t gemm_ldh(const lq_geom &g) { return 256 * ((g.cols + 255) / 256); }
 
-int64_t gemm_workspace_bytes(const lq_geom &g, int64_t ntok) {
-    // room for the tiled form too: tokens padded to a multiple of 16
-    const int64_t xh = (((ntok + 15) / 16 * 16) * gemm_ldh(g) * 2 + 255) & ~(int64_t)255;
-    return xh + ntok * 4;
+// f16 rows of x (padded to a multiple of 16 rows) and their scales
+static int64_t gemm_x_bytes(const lq_geom &g, int64_t ntok) {
+    return lq_align256((ntok + 15) / 16 * 16 * gemm_ldh(g) * 2) + ntok * 4;
 }
 
-// The tiled layout with whole-line stores: workgroup b converts tokens
-// 8 b .. 8 b + 7, one wave each, with the same per-row scale as
-// x_to_f16_kernel, and writes them through LDS 64 value groups at a time. In
-// the 1 KB slice of a 16-token group, the eight tokens' slots of one value
-// octet are 128 contiguous bytes, so every store of the workgroup fills whole
-// 128-byte lines (the one-wave kernel's scattered 16-byte stores wrote twice
-// the bytes). Workgroup (b, y) stores chunks i = y, y + gridDim.y, ... Rows
-// of at most 64 NG groups (NG <= 8); tokens ntok .. of the last 16-token
-// group are written as zeros.
-template <int NG>
-__global__ __launch_bounds__(512) void x_to_f16_tiles_kernel(const float *__restrict__ X, int64_t ldx, int cols,
-                                                             const int32_t *__restrict__ rows_map, int k,
-                                                             int64_t ntok, _Float16 *__restrict__ Xh, int ldh,
-                                                             float *__restrict__ inv, int vec) {
-    __shared__ uint4 stage[64 * 8];   // [lane = 4 quad + octet][token, swizzled]
-    const int lane = lane_id(), tw = wave_id();
-    const int64_t t0 = (int64_t)blockIdx.x * 8, t = t0 + tw;
-    const bool real = t < ntok;
-    const int64_t src = real ? (rows_map ? (int64_t)(rows_map[t] / k) : t) : 0;
-    const float *x = X + src * ldx;
-    const int ngx = cols >> 3, nq = ldh >> 5;
-    lq_f4 lo[NG], hi[NG];
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-        const int gi = lane + 64 * i;
-        lo[i] = hi[i] = lq_f4{0.f, 0.f, 0.f, 0.f};
-        if (real && gi < ngx) {
-            if (vec) {
-                lo[i] = *reinterpret_cast<const lq_f4 *>(x + 8 * gi);
-                hi[i] = *reinterpret_cast<const lq_f4 *>(x + 8 * gi + 4);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    lo[i][c] = x[8 * gi + c];
-                    hi[i][c] = x[8 * gi + 4 + c];
-                }
-            }
-        }
-    }
-    // the largest magnitude as ordered bits; NaN counts as zero (fmaxf's rule)
-    uint32_t mb = 0;
-#pragma unroll
-    for (int i = 0; i < NG; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const float a = lo[i][c], b = hi[i][c];
-            const uint32_t ua = __builtin_bit_cast(uint32_t, a) & 0x7fffffffu;
-            const uint32_t ub = __builtin_bit_cast(uint32_t, b) & 0x7fffffffu;
-            mb = max(mb, max(ua > 0x7f800000u ? 0u : ua, ub > 0x7f800000u ? 0u : ub));
-        }
-    const float m = __builtin_bit_cast(float, wave_max_u32(mb));
-    int s = 0;
-    if (m > 0.0f && m <= 3.4e38f) {
-        int e;
-        frexpf(m, &e);          // m < 2^e <= 2m
-        s = 15 - e;             // m * 2^s in [2^14, 2^15)
-        s = s > 120 ? 120 : s < -120 ? -120 : s;
-    }
-    const float sc = ldexpf(1.0f, s);
-    const int64_t blk0 = (t0 >> 4) * nq;         // 1 KB slice of quad 0 of this 16-token group
-    const int half = (int)((t0 >> 3) & 1);       // tokens 8 half .. 8 half + 7 of the group
-    const int j = threadIdx.x, L = j >> 3, tk = j & 7;   // store: lane L's slot of token tk
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-        if (i % (int)gridDim.y != (int)blockIdx.y) continue;   // this workgroup's share of the chunks
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-        h8 o;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            o[c] = (_Float16)(lo[i][c] * sc);
-            o[4 + c] = (_Float16)(hi[i][c] * sc);
-        }
-        stage[lane * 8 + (tw ^ (lane & 7))] = __builtin_bit_cast(uint4, o);
-        __syncthreads();
-        const int q = 16 * i + (L >> 2);          // quad (32-value slice) of lane L's group
-        if (q < nq) {
-            const int64_t slot = ((blk0 + q) << 6) + 8 * half + tk + 16 * (L & 3);
-            *reinterpret_cast<uint4 *>(Xh + 8 * slot) = stage[L * 8 + (tk ^ (L & 7))];
-        }
-        __syncthreads();
-    }
-    if (real && lane == 0) inv[t] = ldexpf(1.0f, -s);
+int64_t gemm_workspace_bytes(const lq_geom &g, int64_t ntok) {
+    const int64_t x = gemm_x_bytes(g, ntok);
+    const bool tiles = g.type == LQ_Q4_K || g.type == LQ_Q6_K || g.type == LQ_Q8_0;
+    const int64_t split = tiles ? gemm_dense_split_bytes(g, ntok) : 0;
+    return split ? lq_align256(x) + split : x;
 }
 
 int launch_x_to_f16(const float *X, int64_t ldx, int64_t cols, const int32_t *rows_map, int k, int64_t ntok,
-                    _Float16 *Xh, int64_t ldh, float *inv, hipStream_t s, int tiled, float *nrm2) {
+                    _Float16 *Xh, int64_t ldh, float *inv, hipStream_t s, float *nrm2) {
     if (ntok <= 0) return LOCALAI_OK;
-    if (tiled && nrm2) return fail(LOCALAI_EARG, "f16 tiles: no row norms");
     if (cols % 8 || ldh % 8 || ldh < cols) return fail(LOCALAI_EARG, "f16 rows: cols % 8 != 0");
-    if (tiled && ldh % 32) return fail(LOCALAI_EARG, "f16 tiles: row length % 32 != 0");
     const int vec = (uintptr_t)X % 16 == 0 && ldx % 4 == 0;
     const int per = (int)((ldh / 8 + 63) / 64);   // 8-value groups per lane
-    const int64_t npad = tiled ? (ntok + 15) / 16 * 16 : ntok;
-    if (tiled && per <= 8) {
-        // the chunks of an 8-token group split over up to 4 workgroups (each
-        // reads the whole rows for their maxima, mostly from L2), so that
-        // 512 tokens occupy 256 workgroups
-        const dim3 g8((unsigned)(npad / 8), (unsigned)(per < 4 ? per : 4));
-        auto gt = [&](auto kern) {
-            hipLaunchKernelGGL(kern, g8, dim3(512), 0, s, X, ldx, (int)cols, rows_map, k, ntok, Xh, (int)ldh, inv, vec);
-        };
-        if (per <= 1) gt(x_to_f16_tiles_kernel<1>);
-        else if (per <= 2) gt(x_to_f16_tiles_kernel<2>);
-        else if (per <= 4) gt(x_to_f16_tiles_kernel<4>);
-        else gt(x_to_f16_tiles_kernel<8>);
-        LQ_HIP(hipGetLastError());
-        return LOCALAI_OK;
-    }
     // one token per wave; one-wave workgroups below 1024 tokens, so that 512
     // tokens reach every CU (four-wave workgroups left half of them idle)
-    const int wpg = npad < 1024 ? 1 : 4;
-    const dim3 grid((unsigned)((npad + wpg - 1) / wpg));
+    const int wpg = ntok < 1024 ? 1 : 4;
+    const dim3 grid((unsigned)((ntok + wpg - 1) / wpg));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(64 * wpg), 0, s, X, ldx, (int)cols, rows_map, k, ntok, Xh, (int)ldh, inv,
-                           vec, tiled, npad, nrm2);
+                           vec, nrm2);
     };
     if (per <= 1)
         go(x_to_f16_kernel<1>);
@@ -1247,32 +679,17 @@ static int launch_gemm_tile_t(const GemmArgs &a, dim3 grid, hipStream_t s) {
 int launch_gemm(const lq_geom &g, const uint8_t *W, const uint8_t *Wt, const float *X, int64_t ntok, float *Y,
                 int64_t y_ts, int64_t y_rs, void *ws, int64_t ws_bytes, hipStream_t s) {
     if (ntok <= 0) return LOCALAI_OK;
-    if (ws_bytes < gemm_workspace_bytes(g, ntok)) return fail(LOCALAI_EARG, "matmul: workspace too small");
+    if (ws_bytes < gemm_x_bytes(g, ntok)) return fail(LOCALAI_EARG, "matmul: workspace too small");
     const int64_t ldh = gemm_ldh(g);
     _Float16 *Xh = (_Float16 *)ws;
-    float *inv = (float *)((uint8_t *)ws + ((((ntok + 15) / 16 * 16) * ldh * 2 + 255) & ~(int64_t)255));
+    float *inv = (float *)((uint8_t *)ws + lq_align256((ntok + 15) / 16 * 16 * ldh * 2));
     GemmArgs a{};
     a.g = g; a.W = W; a.Xh = Xh; a.ldh = (int)ldh; a.inv = inv; a.ntok = ntok; a.Y = Y; a.y_ts = y_ts; a.y_rs = y_rs;
     a.Wt = Wt;
-    // the CU-tile kernel: Q8_0 tile form, enough tokens to fill the CUs, and
-    // 32-bit byte offsets into the weights and the tiled x
-    const int64_t tiles = (g.rows + MT_ROWS - 1) / MT_ROWS;
-    if (Wt && g.type == LQ_Q8_0 && ntok >= 256 && (size_t)CU_LDS_RESERVE <= max_lds_per_block() &&
-        tiles * mt_nsb(g) * MT_Q80_BLOCK < ((int64_t)1 << 32) && (ntok + 15) / 16 * 16 * ldh * 2 < ((int64_t)1 << 32)) {
-        if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s, 1)) return st;
-        const int64_t nrb = (tiles + CU_RT - 1) / CU_RT, ntb = (ntok + CU_TOKENS - 1) / CU_TOKENS;
-        if (nrb * ntb > ((int64_t)1 << 30)) return fail(LOCALAI_EARG, "matmul: problem too large");
-        const int y_vec = y_rs == 1 && y_ts % 4 == 0 && (uintptr_t)Y % 16 == 0;
-        hipLaunchKernelGGL(gemm_cu_q80_kernel, dim3((unsigned)(nrb * ntb)), dim3(512), CU_LDS_RESERVE, s, a, (int)nrb,
-                           (int)ntb, y_vec);
-        LQ_HIP(hipGetLastError());
-        return LOCALAI_OK;
-    }
     if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
     if (Wt) {
-        const int64_t nwg = ((g.rows + GT_WROWS - 1) / GT_WROWS) * ((ntok + GM_BN - 1) / GM_BN);
-        if (nwg > ((int64_t)1 << 30)) return fail(LOCALAI_EARG, "matmul: problem too large");
-        return launch_gemm_tile_t<GM_DENSE, GM_BN>(a, dim3((unsigned)((nwg + 7) / 8 * 8)), s);
+        const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
+        return launch_gemm_dense(a, (uint8_t *)ws + xb, ws_bytes > xb ? ws_bytes - xb : 0, s);
     }
     const int64_t nwg = ((g.rows + GM_BM - 1) / GM_BM) * ((ntok + GM_BN - 1) / GM_BN);
     if (nwg > ((int64_t)1 << 30)) return fail(LOCALAI_EARG, "matmul: problem too large");

@@ -104,9 +104,9 @@ int64_t gemm_workspace_bytes(const lq_geom &g, int64_t ntok);
 int launch_gemm(const lq_geom &g, const uint8_t *packed, const uint8_t *Wt, const float *x, int64_t ntok, float *y,
                 int64_t y_ts, int64_t y_rs, void *ws, int64_t ws_bytes, hipStream_t s);
 
-// nrm2 (not null, row layout only): each row's sum of squares
+// nrm2 (not null): each row's sum of squares
 int launch_x_to_f16(const float *X, int64_t ldx, int64_t cols, const int32_t *rows_map, int k, int64_t ntok,
-                    _Float16 *Xh, int64_t ldh, float *inv, hipStream_t s, int tiled = 0, float *nrm2 = nullptr);
+                    _Float16 *Xh, int64_t ldh, float *inv, hipStream_t s, float *nrm2 = nullptr);
 // The gate_up expert GEMM's f16 output (GemmArgs::Yh): the down GEMM's input
 // rows and their scales written directly.
 struct MoeF16Out {

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float *__restrict__
     const int t = blockIdx.x * 4 + wave_id();
     if (t >= T) return;
     if constexpr (CONV >= 0)
-        x_to_f16_row<CONV>(t, cv.X, cv.cols, cv.cols, nullptr, 1, T, cv.Xh, cv.ldh, cv.inv, cv.vec, 0, T, cv.nrm2);
+        x_to_f16_row<CONV>(t, cv.X, cv.cols, cv.cols, nullptr, 1, T, cv.Xh, cv.ldh, cv.inv, cv.vec, cv.nrm2);
     route_select_any(logits + (int64_t)t * E, E, k, t, topk_idx, topk_w, MoeTables{}, 0);
 }
 
@@ -1450,7 +1450,7 @@ int launch_moe(const float *h, int64_t T, int64_t H, const float *rw, const floa
         if (gu->g.cols != H || dn->g.cols != I) return fail(LOCALAI_EARG, "moe: expert shapes");
         // gate_up reads the f16 rows of h through the permutation (perm[p] / k)
         if (!h_f16_done)
-            if (int st = launch_x_to_f16(h, H, H, nullptr, 1, T, tb.xh_gu, f16_stride(H), tb.inv_gu, s, 0, tb.hn2))
+            if (int st = launch_x_to_f16(h, H, H, nullptr, 1, T, tb.xh_gu, f16_stride(H), tb.inv_gu, s, tb.hn2))
                 return st;
         // the expert GEMMs read the tile form where there is one (gate_up
         // with inter a multiple of 16), else the row planes

@@ -217,13 +217,18 @@ def check_lds_ring(hipcc: str, flags: list[str], src: Path, kernel: str, per_sta
 
 
 def check_source(hipcc: str, flags: list[str], src: Path, kernel: str, out: Path) -> None:
-    """Compile src to gfx9 assembly and raise if kernel touches a register
-    whose load may still be in flight."""
+    """Compile src to gfx9 assembly and raise if an instantiation of kernel
+    touches a register whose load may still be in flight."""
     cmd = [hipcc, *flags, '--cuda-device-only', '-S', str(src), '-o', str(out)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f'hipcc -S failed for {src.name}:\n{r.stderr[-4000:]}')
-    bad = pending_violations(kernel_lines(out.read_text(), kernel))
-    if bad:
-        shown = '\n'.join(f'  {i}: {why}: {ins}' for i, why, ins in bad[:10])
-        raise RuntimeError(f'{kernel} ({src.name}) touches registers whose loads may still be in flight:\n{shown}')
+    asm = out.read_text()
+    names = sorted(set(re.findall(r'^(_Z\S*' + re.escape(kernel) + r'\S*):', asm, re.M)))
+    if not names:
+        raise RuntimeError(f'{kernel} not found in {src.name}')
+    for name in names:
+        bad = pending_violations(kernel_lines(asm, name))
+        if bad:
+            shown = '\n'.join(f'  {i}: {why}: {ins}' for i, why, ins in bad[:10])
+            raise RuntimeError(f'{name} ({src.name}) touches registers whose loads may still be in flight:\n{shown}')

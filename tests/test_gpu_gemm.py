@@ -91,6 +91,50 @@ def test_q8_0_workgroup_tiles(rows, cols, tokens):
         np.testing.assert_array_equal(gpu_matmul(raw, 8, rows, cols, xs, rows_major=True), got.T)
 
 
+@pytest.mark.parametrize('t', (8, 12, 14))
+@pytest.mark.parametrize('rows,nblocks,tokens', [(16, 1, 1), (257, 2, 17), (272, 5, 49), (300, 6, 81), (40, 16, 113),
+                                                 (512, 24, 130), (8192, 4, 32)])
+def test_dense_tiles_and_splits(t, rows, nblocks, tokens):
+    """The dense kernel's edges: odd and even block counts per split, one and
+    many splits, token tiles of 1 to 8 MFMA tiles, rows past the last row tile;
+    and a workspace with no room for splits (the size of the converted x),
+    which takes one split: the same products, summed in another order."""
+    from localai_amd import _lib, device
+    rng = np.random.default_rng(rows + 31 * nblocks + tokens + t)
+    cols = 256 * nblocks
+    raw = random_ggml(rng, t, rows * cols)
+    xs = rng.standard_normal((tokens, cols)).astype(np.float32)
+    ref = check(gpu_matmul(raw, t, rows, cols, xs), raw, t, rows, cols, xs)
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    xd = device.to_device_f32(xs)
+    torch = device.torch()
+    least = (tokens + 15) // 16 * 16 * cols * 2 + tokens * 4
+    ws = torch.empty(least, dtype=torch.uint8, device=xd.device)
+    y = torch.empty((tokens, rows), dtype=torch.float32, device=xd.device)
+    lib = _lib.load()
+    args = (q.handle, 0, device.ptr(xd), tokens, device.ptr(y), 0, device.ptr(ws))
+    _lib.check(lib.localai_hip_matmul(*args, least, device.stream_ptr()))
+    check(y.cpu().numpy(), raw, t, rows, cols, xs)
+    assert lib.localai_hip_matmul(*args, least - 1, device.stream_ptr()) != 0
+    assert int(lib.localai_hip_matmul_workspace_size(q.handle, tokens)) >= least
+    assert np.isfinite(ref).all()
+    q.close()
+
+
+@pytest.mark.parametrize('t,rows,nblocks,tokens', [(12, 4112, 3, 2000), (14, 4096, 2, 2048), (8, 3900, 4, 2100)])
+def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
+    """More than 256 output tiles: whole rounds (a workgroup's next tile requested
+    before this one's results are stored), none or some tiles left over for
+    the split round, ragged edges; both output layouts hold the same values."""
+    rng = np.random.default_rng(rows + tokens)
+    cols = 256 * nblocks
+    raw = random_ggml(rng, t, rows * cols)
+    xs = rng.standard_normal((tokens, cols)).astype(np.float32)
+    got = gpu_matmul(raw, t, rows, cols, xs)
+    check(got, raw, t, rows, cols, xs)
+    np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
+
+
 def test_rows_major_layout_matches_reference_convention():
     """y_layout 1 is the [rows, tokens] buffer of localai_*_matmul (engine/native_quant.cpp:492)."""
     rng = np.random.default_rng(11)
