@@ -46,6 +46,61 @@ __global__ __launch_bounds__(256) void x_to_f16_kernel(const float *__restrict__
     x_to_f16_row<NG>(t, X, ldx, cols, rows_map, k, ntok, Xh, ldh, inv, vec, nrm2);
 }
 
+// Rows of more than 4096 values: one workgroup per token row, its 256 threads
+// holding the row's 8-value groups (NG each, at most 16384 values) between the
+// maximum and the conversion; the same scale and values as x_to_f16_row. 333
+// rows of 14336 values: 5 us; one wave per row, reading it twice, 19.8 us.
+template <int NG>
+__global__ __launch_bounds__(256) void x_to_f16_wide_kernel(const float *__restrict__ X, int64_t ldx, int cols,
+                                                            const int32_t *__restrict__ rows_map, int k,
+                                                            _Float16 *__restrict__ Xh, int ldh,
+                                                            float *__restrict__ inv, int vec) {
+    __shared__ uint32_t wmax[4];
+    const int64_t t = blockIdx.x;
+    const float *x = X + (rows_map ? (int64_t)(rows_map[t] / k) : t) * ldx;
+    const int ngx = cols >> 3, ng = ldh >> 3;
+    lq_f4 lo[NG], hi[NG];
+    uint32_t mb = 0;
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int gi = threadIdx.x + 256 * i;
+        lo[i] = hi[i] = lq_f4{0.f, 0.f, 0.f, 0.f};
+        if (gi < ngx) {
+            if (vec) {
+                lo[i] = *reinterpret_cast<const lq_f4 *>(x + 8 * gi);
+                hi[i] = *reinterpret_cast<const lq_f4 *>(x + 8 * gi + 4);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    lo[i][c] = x[8 * gi + c];
+                    hi[i][c] = x[8 * gi + 4 + c];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NG; ++i) mb = max(mb, max(f16_mag(lo[i]), f16_mag(hi[i])));
+    mb = wave_max_u32(mb);
+    if (lane_id() == 0) wmax[wave_id()] = mb;
+    __syncthreads();
+    const int s = f16_row_shift(max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+    const float sc = ldexpf(1.0f, s);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int gi = threadIdx.x + 256 * i;
+        if (gi >= ng) continue;
+        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+        h8 o;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            o[c] = (_Float16)(lo[i][c] * sc);
+            o[4 + c] = (_Float16)(hi[i][c] * sc);
+        }
+        *reinterpret_cast<h8 *>(Xh + t * ldh + 8 * gi) = o;
+    }
+    if (threadIdx.x == 0) inv[t] = ldexpf(1.0f, -s);
+}
+
 // ---------------------------------------------------------------- weights
 
 // Exact fp32 values of unit u in unit order (the order of gemv_core.h's x
@@ -630,6 +685,17 @@ int launch_x_to_f16(const float *X, int64_t ldx, int64_t cols, const int32_t *ro
     if (cols % 8 || ldh % 8 || ldh < cols) return fail(LOCALAI_EARG, "f16 rows: cols % 8 != 0");
     const int vec = (uintptr_t)X % 16 == 0 && ldx % 4 == 0;
     const int per = (int)((ldh / 8 + 63) / 64);   // 8-value groups per lane
+    if (per > 8 && per <= 32 && !nrm2) {
+        auto gw = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)ntok), dim3(256), 0, s, X, ldx, (int)cols, rows_map, k, Xh,
+                               (int)ldh, inv, vec);
+        };
+        if (per <= 16) gw(x_to_f16_wide_kernel<4>);
+        else if (per <= 24) gw(x_to_f16_wide_kernel<6>);
+        else gw(x_to_f16_wide_kernel<8>);
+        LQ_HIP(hipGetLastError());
+        return LOCALAI_OK;
+    }
     // one token per wave; one-wave workgroups below 1024 tokens, so that 512
     // tokens reach every CU (four-wave workgroups left half of them idle)
     const int wpg = ntok < 1024 ? 1 : 4;

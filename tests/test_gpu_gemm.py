@@ -135,6 +135,19 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
 
 
+@pytest.mark.parametrize('cols', (4352, 8192, 12544, 16384, 16640))
+def test_long_rows_of_x(cols):
+    """Activation rows past 4096 values (one workgroup per row, each group count)
+    and past 16384 (one wave, read twice), with a row of zeros."""
+    rng = np.random.default_rng(cols)
+    raw = random_ggml(rng, 12, 48 * cols)
+    xs = rng.standard_normal((5, cols)).astype(np.float32)
+    xs[3] = 0.0
+    got = gpu_matmul(raw, 12, 48, cols, xs)
+    check(got, raw, 12, 48, cols, xs)
+    assert not got[3].any()
+
+
 def test_rows_major_layout_matches_reference_convention():
     """y_layout 1 is the [rows, tokens] buffer of localai_*_matmul (engine/native_quant.cpp:492)."""
     rng = np.random.default_rng(11)
