@@ -142,7 +142,12 @@ int localai_hip_matvec_many(int n, const localai_qmat *const *mats, const int64_
 
 /* ---- prefill matmul (MFMA) ---------------------------------------------- */
 
-/* Bytes of device workspace localai_hip_matmul needs for `tokens` rows of x. */
+/* Bytes of device workspace localai_hip_matmul uses for `tokens` rows of x: the
+ * converted rows and, where few output tiles leave room on the chip, partial
+ * sums of a division of K. A workspace with room for the converted rows only
+ * (tokens rounded up to 16, times cols rounded up to 256, 2 bytes each, plus 4
+ * bytes a token) is accepted too: K is then divided less (the sums are taken
+ * in another order). */
 int64_t localai_hip_matmul_workspace_size(const localai_qmat *m, int64_t tokens);
 
 /* Many-token product with matrix `expert` of the handle; counterpart of

@@ -38,9 +38,9 @@ __device__ __forceinline__ void q8_pairs(uint32_t w, lq_h2 d2, uint32_t &lo, uin
     hi = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(lq_h2, h) - off) * d2);
 }
 
-enum { GM_DENSE = 0, GM_MOE_GATE_UP = 1, GM_MOE_DOWN = 2 };
+enum { GM_MOE_GATE_UP = 1, GM_MOE_DOWN = 2 };
 
-// Dense: token tile blockIdx.y of Xh [ntok, ldh]; Y[t * y_ts + r * y_rs].
+// Dense: Xh [ntok, ldh]; Y[t * y_ts + r * y_rs].
 // MoE: work tile blockIdx.y of the expert tile list (expert, first row of
 // the expert-major Xh, valid rows); gate_up writes silu(g) * u to
 // Y[p * y_ts + r] for r < inter, down writes Y[p * y_ts + r].
@@ -188,7 +188,8 @@ __device__ __forceinline__ lq_h8 gt_b(const GtRaw<T> &r, int q, uint32_t pair_ab
     return __builtin_bit_cast(lq_h8, o);
 }
 
-// Dense product of a tile-form handle (gemm_dense.hip): a.Xh / a.inv filled in;
+// Dense product (gemm_dense.hip), a.Wt (Q4_K, Q6_K, Q8_0) or the row planes a.W
+// (Q5_K, Q4_0), a.Xh / a.inv filled in;
 // split_ws: up to split_bytes of scratch for K splits (none: one split)
 int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hipStream_t s);
 int64_t gemm_dense_split_bytes(const lq_geom &g, int64_t ntok);

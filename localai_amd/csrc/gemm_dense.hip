@@ -1,5 +1,5 @@
-// Dense prefill product on f16 MFMA: the K loop that every dense matmul on the
-// tile form runs (contract and arithmetic: gemm.hip).
+// Dense prefill product on f16 MFMA: the kernel that every dense matmul runs
+// (contract and arithmetic: gemm.hip).
 //
 // Workgroup: 8 waves x 2 row tiles (256 weight rows) x 128 tokens (16 NV of
 // them computed), over a range of 256-value blocks of K. Each wave decodes its
@@ -34,15 +34,42 @@ constexpr int GD_RING = 4;             // x steps in LDS
 constexpr int GD_VALU = 32;            // VALU scheduled beside a slice's MFMAs, per half
 constexpr int GD_SLOT = GD_BN * GM_BK * 2;   // bytes of one x step
 
+// Q5_K and Q4_0 handles hold row planes (qformat.h), not the tile form. Any
+// order of K serves a product as long as both operands have it, so lane (row n =
+// lane % 16, c = lane / 16) takes one 16-byte quant piece of its row per step as
+// its K values: piece c % 2 of unit 2 HALF + c / 2 (64 values) of the block,
+// 16 low nibbles and 16 high ones, the operands of slices 0, 1 and 2, 3. The
+// matching 8-value chunk of x is gd_chunk. Q5_K decodes in f32 (its minimum has
+// 17 bits: a packed f16 decode would round twice), about 4.5 VALU per MFMA:
+// 14336 x 4096, 128 tokens 44 us against Q4_K's 33; through an LDS tile of f32
+// decoded weights, 112 workgroups, it took 192.
+template <int T> constexpr bool gd_planes() { return T == LQ_Q5_K || T == LQ_Q4_0; }
+
+// 256-value blocks of a row (x rows are padded with zeros to whole blocks)
+__host__ __device__ inline int64_t gd_blocks(const lq_geom &g) { return (g.cols + 255) / 256; }
+
+// the 8-value chunk (of a step's 16) that lane group q multiplies in slice KK
+template <int T, int KK>
+__device__ __forceinline__ int gd_chunk(int q) {
+    if constexpr (T == LQ_Q5_K) return 8 * (q >> 1) + 4 * (KK >> 1) + 2 * (q & 1) + (KK & 1);
+    else if constexpr (T == LQ_Q4_0) return 8 * (q >> 1) + 4 * (q & 1) + 2 * (KK >> 1) + (KK & 1);
+    else return 4 * KK + q;
+}
+
 // One row tile's weights of one step (128 values), and of one 256-value block
 template <int T> struct GdStep { mt_i4 q; };
 template <> struct GdStep<LQ_Q8_0> { mt_i4 q, p; };
+template <> struct GdStep<LQ_Q4_0> { mt_i4 q; int d; };
 template <int T> struct GdBlock { mt_i4 h; };
 template <> struct GdBlock<LQ_Q6_K> { mt_i4 h, sc; int d; };
+template <> struct GdBlock<LQ_Q5_K> { mt_i4 h, qh; };
+template <> struct GdBlock<LQ_Q4_0> {};
 
 // loads per wave (two row tiles): each step's, each block's
-template <int T> constexpr int gd_step_loads() { return T == LQ_Q8_0 ? 4 : 2; }
-template <int T> constexpr int gd_block_loads() { return T == LQ_Q6_K ? 6 : 2; }
+template <int T> constexpr int gd_step_loads() { return T == LQ_Q8_0 || T == LQ_Q4_0 ? 4 : 2; }
+template <int T> constexpr int gd_block_loads() {
+    return T == LQ_Q6_K ? 6 : T == LQ_Q5_K ? 4 : T == LQ_Q4_0 ? 0 : 2;
+}
 
 __device__ __forceinline__ void cu_load_u16(int &v, const void *base, uint32_t off) {
     asm volatile("global_load_ushort %0, %1, %2" : "=v"(v) : "v"(off), "s"(base) : "memory");
@@ -76,6 +103,8 @@ template <int N, int T>
 __device__ __forceinline__ void gd_wait_step(GdStep<T> (&w)[2]) {
     if constexpr (T == LQ_Q8_0)
         asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0].q), "+v"(w[0].p), "+v"(w[1].q), "+v"(w[1].p) : "n"(N) : "memory");
+    else if constexpr (T == LQ_Q4_0)
+        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0].q), "+v"(w[0].d), "+v"(w[1].q), "+v"(w[1].d) : "n"(N) : "memory");
     else
         asm volatile("s_waitcnt vmcnt(%2)" : "+v"(w[0].q), "+v"(w[1].q) : "n"(N) : "memory");
 }
@@ -85,7 +114,9 @@ __device__ __forceinline__ void gd_wait_block(GdBlock<T> (&b)[2]) {
         asm volatile("s_waitcnt vmcnt(%6)"
                      : "+v"(b[0].h), "+v"(b[0].sc), "+v"(b[0].d), "+v"(b[1].h), "+v"(b[1].sc), "+v"(b[1].d)
                      : "n"(N) : "memory");
-    else
+    else if constexpr (T == LQ_Q5_K)
+        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(b[0].h), "+v"(b[0].qh), "+v"(b[1].h), "+v"(b[1].qh) : "n"(N) : "memory");
+    else if constexpr (T != LQ_Q4_0)
         asm volatile("s_waitcnt vmcnt(%2)" : "+v"(b[0].h), "+v"(b[1].h) : "n"(N) : "memory");
 }
 
@@ -129,6 +160,58 @@ __device__ __forceinline__ GtRaw<T> gd_raw(const GdStep<T> &w, const GdBlock<T> 
     return r;
 }
 
+// Q5_K: f32 scale and minimum {d * sc, dmin * mn} (exact) of the lane's sub-block
+// 4 HALF + 2 (q / 2) + NIB
+template <int HALF, int NIB>
+__device__ __forceinline__ void gd_q5k_scale(const mt_i4 &h, int q, float &a, float &b) {
+    const int o = 16 * (q >> 1) + 8 * NIB;
+    const uint32_t s0 = (uint32_t)h[1], s4 = (uint32_t)h[2], s8 = (uint32_t)h[3];
+    uint32_t sc, mn;
+    if constexpr (HALF == 0) {
+        sc = __builtin_amdgcn_ubfe(s0, o, 6);
+        mn = __builtin_amdgcn_ubfe(s4, o, 6);
+    } else {
+        sc = __builtin_amdgcn_ubfe(s8, o, 4) | (__builtin_amdgcn_ubfe(s0, o + 6, 2) << 4);
+        mn = __builtin_amdgcn_ubfe(s8, o + 4, 4) | (__builtin_amdgcn_ubfe(s4, o + 6, 2) << 4);
+    }
+    a = f16_to_f32((uint32_t)h[0]) * (float)sc;
+    b = f16_to_f32((uint32_t)h[0] >> 16) * (float)mn;
+}
+// Q5_K operand of slice KK: q = nibble | high bit << 4, a value a q - b in one
+// f32 fused multiply-add (exact products, rounded as the row decoders round it),
+// then rounded once to f16
+template <int HALF, int KK>
+__device__ __forceinline__ lq_h8 gd_q5k_b(const mt_i4 &qs, const mt_i4 &qh, int q, float a, float b) {
+    constexpr int nib = KK >> 1, w0 = 2 * (KK & 1);
+    const int bit = 2 * (q >> 1) + 4 * HALF + nib;
+    lq_h8 o;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t lo = ((uint32_t)qs[w0 + i] >> (4 * nib)) & 0x0F0F0F0Fu;
+        const uint32_t hi = ((uint32_t)qh[w0 + i] >> bit) & 0x01010101u;
+        const uint32_t v = lo | (hi << 4);
+        const float f[4] = {__builtin_fmaf(a, ubyte0(v), -b), __builtin_fmaf(a, ubyte1(v), -b),
+                            __builtin_fmaf(a, ubyte2(v), -b), __builtin_fmaf(a, ubyte3(v), -b)};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[4 * i + k] = (_Float16)f[k];
+    }
+    return o;
+}
+// Q4_0 operand of slice KK: q - 8 exactly, times d rounded once
+template <int KK>
+__device__ __forceinline__ lq_h8 gd_q40_b(const mt_i4 &qs, lq_h2 d2) {
+    constexpr int nib = KK >> 1, w0 = 2 * (KK & 1);
+    const lq_h2 k8 = {(_Float16)8.0f, (_Float16)8.0f};
+    uint4 o;
+    auto pair = [&](lq_h2 v) { return __builtin_bit_cast(uint32_t, (v - k8) * d2); };
+    const uint32_t a = ((uint32_t)qs[w0] >> (4 * nib)) & 0x0F0F0F0Fu, b = ((uint32_t)qs[w0 + 1] >> (4 * nib)) & 0x0F0F0F0Fu;
+    o.x = pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(a, 512.0f, false));
+    o.y = pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(a, 512.0f, true));
+    o.z = pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, false));
+    o.w = pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, true));
+    return __builtin_bit_cast(lq_h8, o);
+}
+
 // 1 KB from base + off (per lane) into LDS at the wave-uniform byte address lds
 __device__ __forceinline__ void gd_dma(const void *base, uint32_t off, uint32_t lds) {
     uint32_t keep;
@@ -155,12 +238,18 @@ template <int T, int NV>
 struct GdMain {
     static constexpr int XN = NV / 2;            // x copies per wave and step
     static constexpr int WL = gd_step_loads<T>(), HL = gd_block_loads<T>();
-    static constexpr int BB = mt_block_bytes(T);
+    static constexpr int BB = gd_planes<T>() ? 0 : mt_block_bytes(T);
 
     int lane, wave, nb;
     uint8_t *ring;
     uint32_t ring0, l16, r16;
     const uint8_t *w0p, *w1p;      // the two row tiles at the split's first block
+    // row planes: first row of each row tile in each plane, the lane's row in
+    // the tile, units of a row, the split's first block
+    const uint8_t *pl[2][3];
+    int dr[2], nu, first;
+    int pitch[3];
+    float sa[2], sm[2];            // Q5_K: scale and minimum of the slices' sub-block
     const uint8_t *xb;             // x row p0 at the split's first value
     uint32_t xoff[XN];
     lq_f4 acc[NV][2];
@@ -179,14 +268,43 @@ struct GdMain {
     }
     template <int HALF>
     __device__ __forceinline__ void load_step(GdStep<T> (&d)[2], int b) {
+        if constexpr (gd_planes<T>()) {
+            // the step's first unit (its last valid one past the row's end, whose
+            // weights are then multiplied by a zero scale), its 64-unit chunk
+            int u = 4 * (first + (b < nb ? b : nb - 1)) + 2 * HALF;
+            if (T == LQ_Q4_0) u = u < nu ? u : nu - 1;
+            const int c0 = u & ~63, C = nu - c0 < 64 ? nu - c0 : 64;
+            const int c = lane >> 4;
+            int du = c >> 1;
+            if (T == LQ_Q4_0) du = u + du < nu ? du : 0;
+            const int off = 16 * (du + (c & 1) * C);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                cu_load(d[j].q, pl[j][0] + 16 * (c0 + (int64_t)u), (uint32_t)(dr[j] * pitch[0] + off));
+                if constexpr (T == LQ_Q4_0) cu_load(d[j].d, pl[j][1] + 4 * (int64_t)u, (uint32_t)(dr[j] * pitch[1] + 4 * du));
+            }
+            return;
+        } else {
         const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
         gd_load_step<T, HALF>(d[0], w0p + o, l16);
         gd_load_step<T, HALF>(d[1], w1p + o, l16);
+        }
     }
     __device__ __forceinline__ void load_block(GdBlock<T> (&d)[2], int b) {
-        const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
-        gd_load_block<T>(d[0], w0p + o, l16, r16);
-        gd_load_block<T>(d[1], w1p + o, l16, r16);
+        if constexpr (T == LQ_Q4_0) return;
+        else if constexpr (T == LQ_Q5_K) {
+            const int sb = first + (b < nb ? b : nb - 1), s0 = sb & ~15, nsb = nu >> 2;
+            const int off = 16 * ((lane >> 4) & 1) * (nsb - s0 < 16 ? nsb - s0 : 16);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                cu_load(d[j].qh, pl[j][1] + 16 * (s0 + (int64_t)sb), (uint32_t)(dr[j] * pitch[1] + off));
+                cu_load(d[j].h, pl[j][2] + 16 * (int64_t)sb, (uint32_t)(dr[j] * pitch[2]));
+            }
+        } else {
+            const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
+            gd_load_block<T>(d[0], w0p + o, l16, r16);
+            gd_load_block<T>(d[1], w1p + o, l16, r16);
+        }
     }
     // x operands of slice KK of a slot: token tiles PART * NV / 2 .. into av[PART]
     template <int SLOT, int KK, int PART>
@@ -195,17 +313,29 @@ struct GdMain {
         const uint8_t *xs = ring + SLOT * GD_SLOT + PART * (NV / 2) * 16 * (GM_BK * 2);
 #pragma unroll
         for (int i = 0; i < NV / 2; ++i)
-            av[PART][i] = *reinterpret_cast<const lq_h8 *>(xs + (16 * i + fr) * (GM_BK * 2) + 16 * ((4 * KK + q) ^ fr));
+            av[PART][i] = *reinterpret_cast<const lq_h8 *>(xs + (16 * i + fr) * (GM_BK * 2) + 16 * (gd_chunk<T, KK>(q) ^ fr));
     }
+    // operands of slice KK of half HALF from weight set SET and block header PAR;
+    // b: the slice's block
     template <int SET, int PAR, int HALF, int KK, int DST>
-    __device__ __forceinline__ void decode() {
+    __device__ __forceinline__ void decode(int b) {
         const int q = lane >> 4;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const GtRaw<T> r = gd_raw<T>(w[SET][j], hd[PAR][j]);
-            uint32_t p = 0;
-            if constexpr (T == LQ_Q4_K) p = gd_q4k_pair<HALF, KK>(r.hd);
-            bo[DST][j] = gt_b<T, HALF, KK>(r, q, p);
+            if constexpr (T == LQ_Q5_K) {
+                if constexpr ((KK & 1) == 0) gd_q5k_scale<HALF, (KK >> 1)>(hd[PAR][j].h, q, sa[j], sm[j]);
+                bo[DST][j] = gd_q5k_b<HALF, KK>(w[SET][j].q, hd[PAR][j].qh, q, sa[j], sm[j]);
+            } else if constexpr (T == LQ_Q4_0) {
+                // the scale of the lane's 32-value block; zero past the row's end
+                const uint32_t dd = ((uint32_t)w[SET][j].d >> (16 * (q & 1))) & 0xFFFFu;
+                const uint32_t d = 4 * (first + b) + 2 * HALF + (q >> 1) < nu ? dd * 0x10001u : 0u;
+                bo[DST][j] = gd_q40_b<KK>(w[SET][j].q, __builtin_bit_cast(lq_h2, d));
+            } else {
+                const GtRaw<T> r = gd_raw<T>(w[SET][j], hd[PAR][j]);
+                uint32_t p = 0;
+                if constexpr (T == LQ_Q4_K) p = gd_q4k_pair<HALF, KK>(r.hd);
+                bo[DST][j] = gt_b<T, HALF, KK>(r, q, p);
+            }
         }
     }
     // MFMAs of token tiles PART * NV / 2 .. with the operands bo[SRC]; beside
@@ -230,11 +360,11 @@ struct GdMain {
         __builtin_amdgcn_sched_barrier(0);
     }
     // slice KK of slot S (operands bo[KK % 2], first half of x in av[0]), beside
-    // it the second half of its x and the next slice's operands
+    // it the second half of its x and the next slice's operands (of block bn)
     template <int S, int KK, int SN, int KN, int PN, int HN>
-    __device__ __forceinline__ void slice() {
+    __device__ __forceinline__ void slice(int bn) {
         read_x<S, KK, 1>();
-        if constexpr (SN >= 0) decode<SN, PN, HN, KN, (KK + 1) & 1>();
+        if constexpr (SN >= 0) decode<SN, PN, HN, KN, (KK + 1) & 1>(bn);
         mfmas<KK & 1, 0>();
         if constexpr (SN >= 0) read_x<SN, KN, 0>();
         mfmas<KK & 1, 1>();
@@ -247,14 +377,14 @@ struct GdMain {
         // requests spread over the slices, the weights' registers being those
         // that the previous step decoded: second half of x(s + 2)
         if constexpr (TAIL <= 2) dma<XN / 2, XN>((S + 2) & 3, 2 * b + HALF + 2);
-        slice<S, 0, S, 1, PAR, HALF>();
+        slice<S, 0, S, 1, PAR, HALF>(b);
         if constexpr (TAIL <= 1) {
             // the next block's header (half 0), the weights of step s + 3
             if constexpr (HALF == 0) load_block(hd[PAR ^ 1], b + 1);
             load_step<HN>(w[(S + 3) & 3], b + 1 + HALF);
         }
-        slice<S, 1, S, 2, PAR, HALF>();
-        slice<S, 2, S, 3, PAR, HALF>();
+        slice<S, 1, S, 2, PAR, HALF>(b);
+        slice<S, 2, S, 3, PAR, HALF>(b);
         if constexpr (TAIL < 4) {
             // requested, in order: in step s - 1 the second half of x(s + 1),
             // the next block's header (if its half is 0), the weights of step
@@ -269,7 +399,7 @@ struct GdMain {
             if constexpr (TAIL <= 1) dma<0, XN / 2>((S + 3) & 3, 2 * b + HALF + 3);
             __builtin_amdgcn_sched_barrier(0);
         }
-        slice<S, 3, TAIL < 4 ? SN : -1, 0, PN, HN>();
+        slice<S, 3, TAIL < 4 ? SN : -1, 0, PN, HN>(b + HALF);
     }
     // the first requests of a tile (setup done): what step 0 does not request
     __device__ __forceinline__ void issue() {
@@ -298,7 +428,7 @@ struct GdMain {
         gd_wait_block<0, T>(hd[0]);
         __syncthreads();
         read_x<0, 0, 0>();
-        decode<0, 0, 0, 0, 0>();
+        decode<0, 0, 0, 0, 0>(0);
         int b = 0;
         for (; b + 2 < nb; b += 2) {
             step<0, 0, 0>(b);
@@ -319,14 +449,28 @@ struct GdMain {
     // output tile `tile`, blocks sb0 .. sb0 + n - 1
     __device__ __forceinline__ void setup(const GemmArgs &a, int tile, int ntt, int64_t sb0, int n) {
         const int64_t p0 = (int64_t)(tile % ntt) * GD_BN, t0 = 2 * GD_NW * (int64_t)(tile / ntt) + 2 * wave;
-        const int64_t tiles = (a.g.rows + MT_ROWS - 1) / MT_ROWS, nsb = mt_nsb(a.g);
+        const int64_t tiles = (a.g.rows + MT_ROWS - 1) / MT_ROWS, nsb = gd_blocks(a.g);
         const int tn = (int)(a.ntok - p0 < GD_BN ? a.ntok - p0 : GD_BN);
         fresh_lane();
         l16 = 16 * lane;
         r16 = 16 * (lane & 15);
         nb = n;
-        w0p = a.Wt + ((t0 < tiles ? t0 : tiles - 1) * nsb + sb0) * BB;
-        w1p = a.Wt + ((t0 + 1 < tiles ? t0 + 1 : tiles - 1) * nsb + sb0) * BB;
+        if constexpr (gd_planes<T>()) {
+            first = (int)sb0;
+            nu = (int)a.g.nu;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) pitch[p] = (int)a.g.pitch[p];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int64_t r = (t0 + j < tiles ? t0 + j : tiles - 1) * MT_ROWS;
+                dr[j] = (int)(r + (lane & 15) < a.g.rows ? lane & 15 : a.g.rows - 1 - r);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) pl[j][p] = a.W + a.g.plane[p] + r * a.g.pitch[p];
+            }
+        } else {
+            w0p = a.Wt + ((t0 < tiles ? t0 : tiles - 1) * nsb + sb0) * BB;
+            w1p = a.Wt + ((t0 + 1 < tiles ? t0 + 1 : tiles - 1) * nsb + sb0) * BB;
+        }
         xb = reinterpret_cast<const uint8_t *>(a.Xh + p0 * a.ldh + sb0 * 256);
         // copy i of wave w fills rows 4 (8 i + w) .. + 3 of the step: lane l row
         // + l / 16, position l % 16, from the row's 16-byte chunk
@@ -376,7 +520,7 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
     const GemmArgs &a = d.a;
     const int lane = lane_id(), wave = wave_id();
     const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN);
-    const int nsb = (int)mt_nsb(a.g);
+    const int nsb = (int)gd_blocks(a.g);
     // Workgroups go to the 8 XCDs round robin (id % 8); in every round each XCD
     // takes a contiguous range of the items, so that the token tiles of a row
     // block read its weights from one L2. The round after the whole tiles holds
@@ -509,7 +653,7 @@ struct DensePlan {
 // 183, 4 64.8, 5 (taken) 63.9, 8 98 (two rounds).
 static DensePlan dense_plan(const lq_geom &g, int64_t ntok) {
     DensePlan p;
-    const int64_t nsb = mt_nsb(g);
+    const int64_t nsb = gd_blocks(g);
     p.tiles = (g.rows + GD_BM - 1) / GD_BM * ((ntok + GD_BN - 1) / GD_BN);
     p.full = (int)(p.tiles / 256 * 256);
     p.rest = (int)(p.tiles - p.full);
@@ -537,7 +681,7 @@ int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hi
     constexpr int lds = GD_RING * GD_SLOT;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
     DensePlan p = dense_plan(a.g, a.ntok);
-    if (p.rest) p.fit(mt_nsb(a.g), split_bytes / (p.rest * GD_PART * 4));
+    if (p.rest) p.fit(gd_blocks(a.g), split_bytes / (p.rest * GD_PART * 4));
     // 32-bit byte offsets into the 128 x rows of a workgroup
     if ((int64_t)a.ldh * 2 * GD_BN >= ((int64_t)1 << 32) || p.tiles > ((int64_t)1 << 30))
         return fail(LOCALAI_EARG, "matmul: problem too large");
@@ -545,9 +689,9 @@ int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hi
     const dim3 grid(p.full ? 256 : (unsigned)((p.rest * p.splits + 7) / 8 * 8));
     switch (a.g.type) {
 #define LQ_GD(TT) case TT: hipLaunchKernelGGL(gemm_dense_kernel<TT>, grid, dim3(64 * GD_NW), lds, s, d); break;
-        LQ_GD(LQ_Q4_K) LQ_GD(LQ_Q6_K) LQ_GD(LQ_Q8_0)
+        LQ_GD(LQ_Q4_K) LQ_GD(LQ_Q6_K) LQ_GD(LQ_Q8_0) LQ_GD(LQ_Q5_K) LQ_GD(LQ_Q4_0)
 #undef LQ_GD
-        default: return fail(LOCALAI_ETYPE, "matmul: no tile form for this GGML type");
+        default: return fail(LOCALAI_ETYPE, "matmul: unsupported GGML type");
     }
     LQ_HIP(hipGetLastError());
     if (p.splits > 1) {

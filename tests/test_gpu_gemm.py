@@ -91,7 +91,7 @@ def test_q8_0_workgroup_tiles(rows, cols, tokens):
         np.testing.assert_array_equal(gpu_matmul(raw, 8, rows, cols, xs, rows_major=True), got.T)
 
 
-@pytest.mark.parametrize('t', (8, 12, 14))
+@pytest.mark.parametrize('t', TYPES)
 @pytest.mark.parametrize('rows,nblocks,tokens', [(16, 1, 1), (257, 2, 17), (272, 5, 49), (300, 6, 81), (40, 16, 113),
                                                  (512, 24, 130), (8192, 4, 32)])
 def test_dense_tiles_and_splits(t, rows, nblocks, tokens):
@@ -121,7 +121,8 @@ def test_dense_tiles_and_splits(t, rows, nblocks, tokens):
     q.close()
 
 
-@pytest.mark.parametrize('t,rows,nblocks,tokens', [(12, 4112, 3, 2000), (14, 4096, 2, 2048), (8, 3900, 4, 2100)])
+@pytest.mark.parametrize('t,rows,nblocks,tokens', [(12, 4112, 3, 2000), (14, 4096, 2, 2048), (8, 3900, 4, 2100),
+                                                   (13, 4112, 2, 2000), (2, 4100, 3, 1990)])
 def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     """More than 256 output tiles: whole rounds (a workgroup's next tile requested
     before this one's results are stored), none or some tiles left over for
@@ -133,6 +134,26 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     got = gpu_matmul(raw, t, rows, cols, xs)
     check(got, raw, t, rows, cols, xs)
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
+
+
+@pytest.mark.parametrize('t', (2, 8))
+@pytest.mark.parametrize('cols', (32, 64, 96, 2144, 4128, 4192))
+def test_dense_rows_of_partial_blocks(t, cols):
+    """32-value blocks: rows that end inside a 256-value block or a 64-value unit,
+    around the 4096-value chunks of the row planes; the last block's scale is
+    infinite in one row, whose outputs must not leak into others."""
+    rng = np.random.default_rng(cols + t)
+    rows, tokens = 37, 33
+    raw = random_ggml(rng, t, rows * cols)
+    xs = rng.standard_normal((tokens, cols)).astype(np.float32)
+    got = gpu_matmul(raw, t, rows, cols, xs)
+    check(got, raw, t, rows, cols, xs)
+    b = np.frombuffer(raw, np.uint8).copy().reshape(rows, -1)
+    size = 18 if t == 2 else 34
+    b[5, -size:-size + 2] = (0x00, 0x7c)
+    inf = gpu_matmul(b.tobytes(), t, rows, cols, xs)
+    keep = np.arange(rows) != 5
+    np.testing.assert_array_equal(inf[:, keep], got[:, keep])
 
 
 @pytest.mark.parametrize('cols', (4352, 8192, 12544, 16384, 16640))
