@@ -525,18 +525,32 @@ int launch_matvec_mfma(const lq_geom &g, const uint8_t *Wt, const float *x, floa
 // mt_pass in turn (so y[t] is bit-identical to a one-vector call on x[t]);
 // the next vector's x is requested before the current one is summed. The
 // weights are read from HBM once per call however many vectors there are.
+//
+// The vectors go in groups of MT_TOKS: each wave leaves its part of every
+// vector's sums in LDS and the workgroup meets once per group, all of the
+// group's row sums being added at once (16 RT threads a vector, the waves in
+// order, as mt_pass does). Meeting twice per vector, with 16 RT threads summing
+// while the rest waited, took 3.3 us a vector at 14336 x 4096 Q4_K, of which the
+// arithmetic is about 1.3. The sums alternate between two buffers, so a group's
+// first sums may be written while the last group's are still being added.
+constexpr int MT_TOKS = 4;
+
+__host__ __device__ constexpr size_t mt_tok_lds_bytes(int type, int waves, int spw, int rt) {
+    return (size_t)waves * spw * mt_xbytes(type) + (size_t)2 * MT_TOKS * waves * rt * 64 * 4;
+}
+
 template <int TYPE, int SPW, int RT, int MAXT>
-__global__ __launch_bounds__(MAXT) void gemv_mfma_tok(const uint8_t *__restrict__ Wt, int64_t rows, int nb,
+__global__ __launch_bounds__(MAXT, MAXT == 1024 && SPW * RT == 1 ? 8 : 1) void gemv_mfma_tok(const uint8_t *__restrict__ Wt, int64_t rows, int nb,
                                                       int64_t tiles, const float *__restrict__ x, int64_t ldx,
                                                       float *__restrict__ y, int64_t ldy, int ntok) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int lane = lane_id(), wv = wave_id(), sb0 = wv * SPW, nsb = mt_nsb(nb, sb0, SPW);
+    constexpr int XB = mt_xbytes(TYPE);
+    const int lane = lane_id(), wv = wave_id(), nw = blockDim.x >> 6, sb0 = wv * SPW, nsb = mt_nsb(nb, sb0, SPW);
     const int64_t blk = blockIdx.x;
-    const int i = threadIdx.x;
-    const int64_t tile = blk * RT + ((i >> 4) & (RT - 1)), row = tile * MT_ROWS + (i & 15);
-    const bool mine = i < RT * 16 && tile < tiles && row < rows;
-    float4 xv[1][SPW];
-    mt_load_x<SPW>(xv[0], x, nb, sb0, lane);
+    uint8_t *wl = smem + wv * SPW * XB;
+    float *red = reinterpret_cast<float *>(smem + nw * SPW * XB);   // [2][MT_TOKS][nw][RT][64]
+    float4 xv[SPW];
+    mt_load_x<SPW>(xv, x, nb, sb0, lane);
     MtW<TYPE> w[RT][SPW];
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
@@ -544,14 +558,42 @@ __global__ __launch_bounds__(MAXT) void gemv_mfma_tok(const uint8_t *__restrict_
         mt_load_tile<TYPE, SPW>(w[t], Wt + tl * nb * mt_block_bytes(TYPE), nb, sb0, nsb, lane);
     }
     __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0; t < ntok; ++t) {
-        float4 xn[SPW];
-        mt_load_x<SPW>(xn, x + (int64_t)(t + 1 < ntok ? t + 1 : t) * ldx, nb, sb0, lane);
-        float *fin;
-        mt_pass<TYPE, SPW, RT, 1>(w, xv, nsb, smem, fin);
-        if (mine) y[(int64_t)t * ldy + row] = fin[i];
+    const MtLane<TYPE> L = mt_lane<TYPE>(lane);
+    for (int t0 = 0; t0 < ntok; t0 += MT_TOKS) {
+        const int nt = ntok - t0 < MT_TOKS ? ntok - t0 : MT_TOKS;
+        float *buf = red + (t0 / MT_TOKS & 1) * MT_TOKS * nw * RT * 64;
+        for (int j = 0; j < nt; ++j) {
+            // the wave's own region: its reads of the last vector precede these
+            // writes in its LDS order
 #pragma unroll
-        for (int k = 0; k < SPW; ++k) xv[0][k] = xn[k];
+            for (int k = 0; k < SPW; ++k) mt_stage<TYPE>(xv[k], wl + k * XB, lane);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const int tn = t0 + j + 1 < ntok ? t0 + j + 1 : ntok - 1;
+            mt_load_x<SPW>(xv, x + (int64_t)tn * ldx, nb, sb0, lane);
+            float acc[RT];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < SPW; ++k) {
+                if (k >= nsb) break;
+                const MtA<TYPE> a = mt_load_a<TYPE>(wl + k * XB, L);
+#pragma unroll
+                for (int t = 0; t < RT; ++t) acc[t] = mt_dot<TYPE>(w[t][k], a, L, acc[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) buf[((j * nw + wv) * RT + t) * 64 + lane] = acc[t];
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < nt * RT * 16; i += blockDim.x) {
+            const int j = i / (RT * 16), t = (i >> 4) & (RT - 1), n = i & 15;
+            float s = 0.0f;
+            for (int kk = 0; kk < nw; ++kk) {
+                const float *r = buf + ((j * nw + kk) * RT + t) * 64 + n;
+                s += (r[0] + r[16]) + (r[32] + r[48]);
+            }
+            const int64_t tile = blk * RT + t, row = tile * MT_ROWS + n;
+            if (tile < tiles && row < rows) y[(int64_t)(t0 + j) * ldy + row] = s;
+        }
     }
 }
 
@@ -565,14 +607,30 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
     if (nb > 72) return fail(LOCALAI_EARG, "mfma matvec: K too large (more than 18432 values)");
     const bool q6 = g.type == LQ_Q6_K, q8 = g.type == LQ_Q8_0;
     const int64_t tiles = (g.rows + MT_ROWS - 1) / MT_ROWS;
-    // up to 32 super-blocks: up to 16 waves (SPW = ceil(nb / 16)), two Q4_K
-    // tiles per workgroup where one super-block per wave leaves room, as in
-    // the one-vector plan; longer rows: 8 waves of ceil(nb / 8) blocks (up to
-    // 9 for K <= 18432), which fit in registers only below 16 waves
+    // up to 32 super-blocks: up to 16 waves (SPW = ceil(nb / 16)), as in the
+    // one-vector plan; longer rows: 8 waves of ceil(nb / 8) blocks (up to 9 for
+    // K <= 18432), which fit in registers only below 16 waves
     const int spw = nb <= 32 ? (nb + 15) / 16 : (nb + 7) / 8, waves = (nb + spw - 1) / spw;
-    const int rt = spw == 1 && tiles >= 768 && !q6 ? 2 : 1;
+    // Row tiles per workgroup: a vector costs a wave about 82 instructions of
+    // staging and 35 a tile, and a CU one workgroup of 2 or 4 tiles at a time (two
+    // of one tile take as long as one after the other). More tiles share the
+    // staging as long as the workgroups still fill the CUs: 14336 x 4096 Q4_K, 31
+    // vectors: 1 tile 95.1 us, 2 65.2, 4 54.9; 4096 x 4096, 4 vectors: 7.0, 7.8,
+    // 12.2. Four tiles are left out for Q6_K (registers: 32000 rows, 7 vectors,
+    // 53.9 us against 49.5 with two) and below four vectors (14336 rows, 2
+    // vectors: 12.6 against 11.6), more than one where a wave has several blocks
+    // (4096 x 8192, 7 vectors: 24.4 against 16.0).
+    int rt = 1;
+    int64_t best = (tiles + 255) / 256 * (82 + 35);
+    for (int r = 2; spw == 1 && r <= (q6 || ntok < 4 ? 2 : 4); r *= 2) {
+        const int64_t cost = (tiles + 256 * r - 1) / (256 * r) * (82 + 35 * r);
+        if (cost < best) {
+            best = cost;
+            rt = r;
+        }
+    }
     dim3 grid((unsigned)((tiles + rt - 1) / rt)), block(64 * waves);
-    const size_t lds = mt_lds_bytes(g.type, waves, spw, 1, rt);
+    const size_t lds = mt_tok_lds_bytes(g.type, waves, spw, rt);
 #define MT_T(S, R, M)                                                                                          \
     do {                                                                                                       \
         if (q6) hipLaunchKernelGGL((gemv_mfma_tok<LQ_Q6_K, S, R, M>), grid, block, lds, s, Wt, g.rows, nb, tiles, x, \
@@ -582,9 +640,20 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
         else hipLaunchKernelGGL((gemv_mfma_tok<LQ_Q4_K, S, R, M>), grid, block, lds, s, Wt, g.rows, nb, tiles, x, ldx, \
                                 y, ldy, ntok);                                                                 \
     } while (0)
+#define MT_T4(M)                                                                                              \
+    do {                                                                                                       \
+        if (q8) hipLaunchKernelGGL((gemv_mfma_tok<LQ_Q8_0, 1, 4, M>), grid, block, lds, s, Wt, g.rows, nb, tiles, x, \
+                                   ldx, y, ldy, ntok);                                                         \
+        else hipLaunchKernelGGL((gemv_mfma_tok<LQ_Q4_K, 1, 4, M>), grid, block, lds, s, Wt, g.rows, nb, tiles, x, ldx, \
+                                y, ldy, ntok);                                                                 \
+    } while (0)
     switch (spw) {
-        case 1: if (rt == 2) MT_T(1, 2, 1024); else MT_T(1, 1, 1024); break;
-        case 2: MT_T(2, 1, 1024); break;
+        case 1:
+            if (rt == 4) MT_T4(1024);
+            else if (rt == 2) MT_T(1, 2, 1024);
+            else MT_T(1, 1, 1024);
+            break;
+                case 2: MT_T(2, 1, 1024); break;
         case 5: MT_T(5, 1, 512); break;
         case 6: MT_T(6, 1, 512); break;
         case 7: MT_T(7, 1, 512); break;
@@ -592,6 +661,7 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
         default: MT_T(9, 1, 512); break;
     }
 #undef MT_T
+#undef MT_T4
     LQ_HIP(hipGetLastError());
     return LOCALAI_OK;
 }

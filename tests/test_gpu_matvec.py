@@ -122,6 +122,27 @@ def test_multi_vector_on_the_tile_form(t, rows, cols, ntok):
     q.close()
 
 
+@pytest.mark.parametrize('t', (12, 14, 8))
+@pytest.mark.parametrize('rows,nsb,ntok', [(16 * 260 - 3, 3, 6), (16 * 600 + 5, 2, 9), (16 * 780, 1, 31), (16 * 1100 + 1, 2, 4),
+                                           (40, 1, 13)])
+def test_multi_vector_groups_and_row_tiles(t, rows, nsb, ntok):
+    """Vector counts around the groups of four, one, two and four row tiles per
+    workgroup, ragged last tiles: each y[t] equals the one-vector call bit
+    for bit."""
+    from localai_amd import device
+    rng = np.random.default_rng(rows + nsb + ntok + t)
+    cols = 256 * nsb
+    raw = random_ggml(rng, t, rows * cols)
+    x = rng.standard_normal((ntok, cols)).astype(np.float32)
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    xd = device.to_device_f32(x)
+    got = q.matvec(xd).cpu().numpy()
+    for i in range(ntok):
+        one = q.matvec(xd[i].contiguous()).cpu().numpy()
+        np.testing.assert_array_equal(got[i].view(np.uint32), one.view(np.uint32))
+    q.close()
+
+
 @pytest.mark.parametrize('name,t,rows,cols', [
     ('ffn_gate', 12, 14336, 4096), ('ffn_down', 14, 4096, 14336), ('attn_v', 14, 1024, 4096),
     ('attn_k', 12, 1024, 4096)])
