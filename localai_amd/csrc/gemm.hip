@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void x_to_f16_kernel(const float *__restrict__
 // Rows of more than 4096 values: one workgroup per token row, its 256 threads
 // holding the row's 8-value groups (NG each, at most 16384 values) between the
 // maximum and the conversion; the same scale and values as x_to_f16_row. 333
-// rows of 14336 values: 5 us; one wave per row, reading it twice, 19.8 us.
+// rows of 14336 values: 6.9 us; one wave per row, reading it twice, 19.8 us.
 template <int NG>
 __global__ __launch_bounds__(256) void x_to_f16_wide_kernel(const float *__restrict__ X, int64_t ldx, int cols,
                                                             const int32_t *__restrict__ rows_map, int k,
@@ -681,8 +681,8 @@ int launch_gemm(const lq_geom &g, const uint8_t *W, const uint8_t *Wt, const flo
     GemmArgs a{};
     a.g = g; a.W = W; a.Xh = Xh; a.ldh = (int)ldh; a.inv = inv; a.ntok = ntok; a.Y = Y; a.y_ts = y_ts; a.y_rs = y_rs;
     a.Wt = Wt;
-    if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
     const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
+    if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
     return launch_gemm_dense(a, (uint8_t *)ws + xb, ws_bytes > xb ? ws_bytes - xb : 0, s);
 }
 
