@@ -44,10 +44,13 @@ __global__ __launch_bounds__(256) void x_to_f16_kernel(const float *__restrict__
     x_to_f16_row<NG>(t, X, ldx, cols, rows_map, k, ntok, Xh, ldh, inv, vec, nrm2);
 }
 
-// Rows of more than 4096 values: one workgroup per token row, its 256 threads
+// Rows of more than 2048 values: one workgroup per token row, its 256 threads
 // holding the row's 8-value groups (NG each, at most 16384 values) between the
 // maximum and the conversion; the same scale and values as x_to_f16_row. 333
-// rows of 14336 values: 6.9 us; one wave per row, reading it twice, 19.8 us.
+// rows of 14336 values: 6.9 us; one wave per row, reading it twice, 19.8 us. A
+// wave per row holds 4096 values too, but its eight loads a lane are latency: the
+// 77-token product of 4096 x 4096 23.3 -> 22.7 us, 1000 tokens 36.9 -> 36.5; at
+// 1024 values the wave per row is ahead (26.4 us against 26.5).
 template <int NG>
 __global__ __launch_bounds__(256) void x_to_f16_wide_kernel(const float *__restrict__ X, int64_t ldx, int cols,
                                                             const int32_t *__restrict__ rows_map, int k,
@@ -614,12 +617,13 @@ int launch_x_to_f16(const float *X, int64_t ldx, int64_t cols, const int32_t *ro
     if (cols % 8 || ldh % 8 || ldh < cols) return fail(LOCALAI_EARG, "f16 rows: cols % 8 != 0");
     const int vec = (uintptr_t)X % 16 == 0 && ldx % 4 == 0;
     const int per = (int)((ldh / 8 + 63) / 64);   // 8-value groups per lane
-    if (per > 8 && per <= 32 && !nrm2) {
+    if (per > 4 && per <= 32 && !nrm2) {
         auto gw = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3((unsigned)ntok), dim3(256), 0, s, X, ldx, (int)cols, rows_map, k, Xh,
                                (int)ldh, inv, vec);
         };
-        if (per <= 16) gw(x_to_f16_wide_kernel<4>);
+        if (per <= 8) gw(x_to_f16_wide_kernel<2>);
+        else if (per <= 16) gw(x_to_f16_wide_kernel<4>);
         else if (per <= 24) gw(x_to_f16_wide_kernel<6>);
         else gw(x_to_f16_wide_kernel<8>);
         LQ_HIP(hipGetLastError());

@@ -644,13 +644,14 @@ struct DensePlan {
 };
 
 // A workgroup per CU: whole rounds of 256 tiles, then the rest split in K over
-// one more round. A 256-value block costs a workgroup 1.2 us (32 tokens) to 3.2
-// us (128) beside 7 us of launch, first loads and stores, while parts write and
-// read their sums (3.5 TB/s for both ways together) and need the summing launch
-// (3.5 us): the split with the least total. Measured, whole calls: 4096 x 4096
-// Q4_K, 77 tokens: 1 part 49.6 us, 4 23.8, 8 (taken) 22.3, 16 25.2; 14336 x
-// 4096, 256 tokens: 1 56.9, 2 (taken) 45.8; 4096 x 14336 Q6_K, 333 tokens: 1
-// 183, 4 64.8, 5 (taken) 63.9, 8 98 (two rounds).
+// one more round. A 256-value block costs a workgroup 0.9 us (32 tokens), 1.9 (96)
+// or 3.2 (128: bound by its MFMAs and decode, the others by latency), while parts
+// write and read their sums (3.5 TB/s for both ways together) and need the
+// summing launch (5 us, 1.5 more for every further eight parts it adds up): the
+// split with the least total. Measured, whole calls: 4096 x 4096 Q4_K, 77 tokens:
+// 1 part 49.6 us, 4 23.8, 8 (taken) 22.3, 16 25.2; 14336 x 4096, 256 tokens: 1
+// 56.9, 2 (taken) 45.8; 4096 x 14336 Q6_K, 333 tokens: 1 183, 4 64.8, 5 (taken)
+// 63.9, 8 98 (two rounds); 14080 x 1280, 120 tokens: 1 (taken) 25.3, 3 26.9.
 static DensePlan dense_plan(const lq_geom &g, int64_t ntok) {
     DensePlan p;
     const int64_t nsb = gd_blocks(g);
@@ -659,13 +660,13 @@ static DensePlan dense_plan(const lq_geom &g, int64_t ntok) {
     p.rest = (int)(p.tiles - p.full);
     p.splits = 1;
     const int64_t nv = ntok >= GD_BN ? 8 : (ntok + 31) / 32 * 2;
-    const double block_us = 0.55 + 0.33 * (double)nv;
+    const double block_us = nv == 8 ? 3.2 : 0.4 + 0.25 * (double)nv;
     const double part_us = (double)(ntok < GD_BN ? ntok : GD_BN) * GD_BM * 4.0 / 3.5e6;
     double best = 0.0;
     for (int64_t s = 1; p.rest && s <= nsb && s * p.rest <= 256; ++s) {
         const int64_t blocks = (nsb + s - 1) / s;
         if ((nsb + blocks - 1) / blocks != s) continue;
-        const double us = block_us * (double)blocks + (s > 1 ? 3.5 + (double)(s * p.rest) * part_us : 0.0);
+        const double us = block_us * (double)blocks + (s > 1 ? 5.0 + 1.5 * (double)((s - 1) / 8) + (double)(s * p.rest) * part_us : 0.0);
         if (s == 1 || us < best) {
             best = us;
             p.splits = (int)s;

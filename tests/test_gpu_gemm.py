@@ -156,9 +156,9 @@ def test_dense_rows_of_partial_blocks(t, cols):
     np.testing.assert_array_equal(inf[:, keep], got[:, keep])
 
 
-@pytest.mark.parametrize('cols', (4352, 8192, 12544, 16384, 16640))
+@pytest.mark.parametrize('cols', (2304, 4096, 4352, 8192, 12544, 16384, 16640))
 def test_long_rows_of_x(cols):
-    """Activation rows past 4096 values (one workgroup per row, each group count)
+    """Activation rows past 2048 values (one workgroup per row, each group count)
     and past 16384 (one wave, read twice), with a row of zeros."""
     rng = np.random.default_rng(cols)
     raw = random_ggml(rng, 12, 48 * cols)
