@@ -41,7 +41,7 @@ constexpr int GD_SLOT = GD_BN * GM_BK * 2;   // bytes of one x step
 // 16 low nibbles and 16 high ones, the operands of slices 0, 1 and 2, 3. The
 // matching 8-value chunk of x is gd_chunk. Q5_K decodes in f32 (its minimum has
 // 17 bits: a packed f16 decode would round twice), about 4.5 VALU per MFMA:
-// 14336 x 4096, 128 tokens 44 us against Q4_K's 33; through an LDS tile of f32
+// 14336 x 4096, 128 tokens 43 us against Q4_K's 33; through an LDS tile of f32
 // decoded weights, 112 workgroups, it took 192.
 template <int T> constexpr bool gd_planes() { return T == LQ_Q5_K || T == LQ_Q4_0; }
 
@@ -184,7 +184,16 @@ template <int HALF, int KK>
 __device__ __forceinline__ lq_h8 gd_q5k_b(const mt_i4 &qs, const mt_i4 &qh, int q, float a, float b) {
     constexpr int nib = KK >> 1, w0 = 2 * (KK & 1);
     const int bit = 2 * (q >> 1) + 4 * HALF + nib;
-    lq_h8 o;
+    // two f32 to f16, rounded to nearest even, the f32 values opaque: seen
+    // together, the compiler fused half of the multiply-adds with their
+    // conversion into v_fma_mix{lo,hi}_f16, which take twice as long and do not
+    // hide under the MFMAs (14336 x 4096, 1024 tokens: 161.9 us against 156.0)
+    auto pack = [](float x, float y) {
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        asm("" : "+v"(x), "+v"(y));
+        return (int)__builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, lq_h2));
+    };
+    mt_i4 o;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const uint32_t lo = ((uint32_t)qs[w0 + i] >> (4 * nib)) & 0x0F0F0F0Fu;
@@ -192,10 +201,10 @@ __device__ __forceinline__ lq_h8 gd_q5k_b(const mt_i4 &qs, const mt_i4 &qh, int 
         const uint32_t v = lo | (hi << 4);
         const float f[4] = {__builtin_fmaf(a, ubyte0(v), -b), __builtin_fmaf(a, ubyte1(v), -b),
                             __builtin_fmaf(a, ubyte2(v), -b), __builtin_fmaf(a, ubyte3(v), -b)};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) o[4 * i + k] = (_Float16)f[k];
+        o[2 * i] = pack(f[0], f[1]);
+        o[2 * i + 1] = pack(f[2], f[3]);
     }
-    return o;
+    return __builtin_bit_cast(lq_h8, o);
 }
 // Q4_0 operand of slice KK: q - 8 exactly, times d rounded once
 template <int KK>
