@@ -124,7 +124,9 @@ int localai_hip_qmat_dequant(const localai_qmat *m, int64_t expert, float *out_d
  * fp32 (normwise error about 1e-6); from 2048 row tiles one workgroup per CU
  * loops over the tiles (same arithmetic, same bits). 2..31 vectors of such
  * a handle: the same arithmetic per vector over the tile form, the weights
- * read once per call (each y[t] equal to the one-vector call on x[t]). Other
+ * read once per call (each y[t] equal to the one-vector call on x[t], except
+ * that below 768 row tiles rows of 9 to 32 blocks of 256 are divided over more
+ * waves than for one vector, so their partial sums add up in another order). Other
  * types: fp32 products of exactly decoded weights, fp32 accumulation (the
  * vectors two per launch while cols <= 8192, one otherwise). */
 int localai_hip_matvec(const localai_qmat *m, int64_t expert, const float *x_dev,

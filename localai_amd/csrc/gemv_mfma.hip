@@ -522,7 +522,8 @@ int launch_matvec_mfma(const lq_geom &g, const uint8_t *Wt, const float *x, floa
 // Several vectors, one matrix: y[t] = W x[t] for t < ntok. The workgroup's
 // row tiles are loaded into registers once (every block of the wave at
 // once) and each vector goes through the single-vector arithmetic of
-// mt_pass in turn (so y[t] is bit-identical to a one-vector call on x[t]);
+// mt_pass in turn (so y[t] is bit-identical to a one-vector call on x[t] where
+// both plans divide K over the waves alike);
 // the next vector's x is requested before the current one is summed. The
 // weights are read from HBM once per call however many vectors there are.
 //

@@ -169,6 +169,37 @@ def test_long_rows_of_x(cols):
     assert not got[3].any()
 
 
+@pytest.mark.parametrize('t,rows,nblocks,tokens', [(12, 512, 16, 77), (13, 300, 9, 40)])
+def test_dense_parts_replayed_from_a_graph(t, rows, nblocks, tokens):
+    """A product in several parts of K, captured and replayed with eager work
+    between the replays: every replay equals the eager call bit for bit."""
+    from localai_amd import device
+    torch = device.torch()
+    rng = np.random.default_rng(rows + tokens)
+    cols = 256 * nblocks
+    q = device.QMat.from_ggml(random_ggml(rng, t, rows * cols), t, rows, cols)
+    x = device.to_device_f32(rng.standard_normal((tokens, cols)).astype(np.float32))
+    want = q.matmul(x).clone()
+    out = torch.empty_like(want)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        q.matmul(x, out=out)
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q.matmul(x, out=out)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        q.matmul(x[:17].contiguous())
+        torch.cuda.synchronize()
+    q.close()
+
+
 def test_rows_major_layout_matches_reference_convention():
     """y_layout 1 is the [rows, tokens] buffer of localai_*_matmul (engine/native_quant.cpp:492)."""
     rng = np.random.default_rng(11)
