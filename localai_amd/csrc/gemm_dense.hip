@@ -243,6 +243,19 @@ struct DenseArgs {
 };
 constexpr int64_t GD_PART = GD_BM * GD_BN;
 
+// Order of the output tiles: groups of GD_TG token tiles, in a group the token
+// tiles of a row block side by side, so that the 32 tiles an XCD computes at a
+// time (4 x 8) share both x and weights in its L2. All token tiles of a row block
+// side by side, groups of eight, of four: 14336 x 4096 Q4_K, 2048 tokens 254, 245,
+// 247 us; 28000 x 2048, 1500 tokens 211, 207, 204 us.
+constexpr int GD_TG = 4;
+__device__ __forceinline__ void gd_tile(int tile, int ntt, int nrb, int &rb, int &tt) {
+    const int grp = tile / (GD_TG * nrb), r = tile - grp * GD_TG * nrb;
+    const int gs = ntt - GD_TG * grp < GD_TG ? ntt - GD_TG * grp : GD_TG;
+    rb = r / gs;
+    tt = GD_TG * grp + r % gs;
+}
+
 template <int T, int NV>
 struct GdMain {
     static constexpr int XN = NV / 2;            // x copies per wave and step
@@ -455,9 +468,9 @@ struct GdMain {
         // free may outlive the loop
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    // output tile `tile`, blocks sb0 .. sb0 + n - 1
-    __device__ __forceinline__ void setup(const GemmArgs &a, int tile, int ntt, int64_t sb0, int n) {
-        const int64_t p0 = (int64_t)(tile % ntt) * GD_BN, t0 = 2 * GD_NW * (int64_t)(tile / ntt) + 2 * wave;
+    // output tile (row block rb, token tile tt), blocks sb0 .. sb0 + n - 1
+    __device__ __forceinline__ void setup(const GemmArgs &a, int rb, int tt, int64_t sb0, int n) {
+        const int64_t p0 = (int64_t)tt * GD_BN, t0 = 2 * GD_NW * (int64_t)rb + 2 * wave;
         const int64_t tiles = (a.g.rows + MT_ROWS - 1) / MT_ROWS, nsb = gd_blocks(a.g);
         const int tn = (int)(a.ntok - p0 < GD_BN ? a.ntok - p0 : GD_BN);
         fresh_lane();
@@ -494,10 +507,10 @@ struct GdMain {
     // D: the lane holds token lane % 16 of token tile i and rows 4 (lane / 16) +
     // v of row tile j: one 16-byte store where rows are contiguous. out points
     // at the tile's first row and token
-    __device__ __forceinline__ void store(const GemmArgs &a, int tile, int ntt, float *out, int64_t ts, int64_t rs) {
+    __device__ __forceinline__ void store(const GemmArgs &a, int rb, int tt, float *out, int64_t ts, int64_t rs) {
         fresh_lane();
         const int fr = lane & 15, q = lane >> 4;
-        const int64_t p0 = (int64_t)(tile % ntt) * GD_BN, r0 = (int64_t)(tile / ntt) * GD_BM;
+        const int64_t p0 = (int64_t)tt * GD_BN, r0 = (int64_t)rb * GD_BM;
         const int tn = (int)(a.ntok - p0 < GD_BN ? a.ntok - p0 : GD_BN);
         const int rn = (int)(a.g.rows - r0 < GD_BM ? a.g.rows - r0 : GD_BM);
         const bool vec = rs == 1 && ts % 4 == 0 && (uintptr_t)out % 16 == 0;
@@ -528,11 +541,10 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
     extern __shared__ __attribute__((aligned(16))) uint8_t gd_lds[];
     const GemmArgs &a = d.a;
     const int lane = lane_id(), wave = wave_id();
-    const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN);
+    const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN), nrb = (int)((a.g.rows + GD_BM - 1) / GD_BM);
     const int nsb = (int)gd_blocks(a.g);
     // Workgroups go to the 8 XCDs round robin (id % 8); in every round each XCD
-    // takes a contiguous range of the items, so that the token tiles of a row
-    // block read its weights from one L2. The round after the whole tiles holds
+    // takes a contiguous range of the items (gd_tile's order). The round after the whole tiles holds
     // the rest's parts, ordered (part, tile).
     const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
     const int parts = d.rest * d.splits, pp = (parts + 7) / 8;
@@ -546,24 +558,25 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
         m.ring = gd_lds;
         m.ring0 = (uint32_t)(uintptr_t)gd_lds;
         // item: a whole tile of round base / 256, or this workgroup's part
-        int base = 0, tile, sp;
+        int base = 0, tile, sp, rb, tt;
         bool whole;
         auto item = [&]() {
             whole = base < d.full;
             tile = whole ? base + 32 * xcd + idx : d.full + part % d.rest;
             sp = whole ? 0 : part / d.rest;
+            gd_tile(tile, ntt, nrb, rb, tt);
         };
         auto start = [&]() {
             const int sb0 = whole ? 0 : sp * d.blocks;
             const int nb = whole ? nsb : nsb - sb0 < d.blocks ? nsb - sb0 : d.blocks;
-            m.setup(a, tile, ntt, sb0, nb);
+            m.setup(a, rb, tt, sb0, nb);
             m.issue();
         };
         item();
         start();
         for (;;) {
             m.run();
-            const int tile0 = tile, sp0 = sp;
+            const int tile0 = tile, sp0 = sp, rb0 = rb, tt0 = tt;
             const bool to_y = whole || d.splits == 1;
             base += 256;
             const bool more = base < d.full || (base == d.full && d.full > 0 && part >= 0);
@@ -575,11 +588,9 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
                 start();
             }
             if (to_y)
-                m.store(a, tile0, ntt,
-                        a.Y + (int64_t)(tile0 % ntt) * GD_BN * a.y_ts + (int64_t)(tile0 / ntt) * GD_BM * a.y_rs,
-                        a.y_ts, a.y_rs);
+                m.store(a, rb0, tt0, a.Y + (int64_t)tt0 * GD_BN * a.y_ts + (int64_t)rb0 * GD_BM * a.y_rs, a.y_ts, a.y_rs);
             else
-                m.store(a, tile0, ntt, d.P + ((int64_t)sp0 * d.rest + (tile0 - d.full)) * GD_PART,
+                m.store(a, rb0, tt0, d.P + ((int64_t)sp0 * d.rest + (tile0 - d.full)) * GD_PART,
                         a.y_rs == 1 ? GD_BM : 1, a.y_rs == 1 ? 1 : GD_BN);
             if (!more) break;
         }
@@ -589,7 +600,9 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
     } else {
         // one item per workgroup: only the MFMA tiles that hold tokens
         if (part < 0) return;
-        const int64_t left = a.ntok - (int64_t)((part % d.rest) % ntt) * GD_BN;
+        int rb, tt;
+        gd_tile(part % d.rest, ntt, nrb, rb, tt);
+        const int64_t left = a.ntok - (int64_t)tt * GD_BN;
         const int nv = __builtin_amdgcn_readfirstlane((int)((left + 15) >> 4));
         if (nv <= 2) go(std::integral_constant<int, 2>{});
         else if (nv <= 4) go(std::integral_constant<int, 4>{});
@@ -602,8 +615,10 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
 // blockIdx.x, 16 of its 128 tokens or 32 of its 256 rows, whichever runs slowest)
 __global__ __launch_bounds__(256) void gemm_split_sum_kernel(DenseArgs d) {
     const GemmArgs &a = d.a;
-    const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN), tile = d.full + (int)blockIdx.x;
-    const int64_t p0 = (int64_t)(tile % ntt) * GD_BN, r0 = (int64_t)(tile / ntt) * GD_BM;
+    const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN), nrb = (int)((a.g.rows + GD_BM - 1) / GD_BM);
+    int rb, tt;
+    gd_tile(d.full + (int)blockIdx.x, ntt, nrb, rb, tt);
+    const int64_t p0 = (int64_t)tt * GD_BN, r0 = (int64_t)rb * GD_BM;
     const int tn = (int)(a.ntok - p0 < GD_BN ? a.ntok - p0 : GD_BN);
     const int rn = (int)(a.g.rows - r0 < GD_BM ? a.g.rows - r0 : GD_BM);
     // slow x fast: tokens x rows, or rows x tokens
