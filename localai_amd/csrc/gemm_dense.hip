@@ -544,8 +544,8 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
     const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN), nrb = (int)((a.g.rows + GD_BM - 1) / GD_BM);
     const int nsb = (int)gd_blocks(a.g);
     // Workgroups go to the 8 XCDs round robin (id % 8); in every round each XCD
-    // takes a contiguous range of the items (gd_tile's order). The round after the whole tiles holds
-    // the rest's parts, ordered (part, tile).
+    // takes a contiguous range of the items (gd_tile's order). The round after the
+    // whole tiles holds the rest's parts, ordered (part, tile).
     const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
     const int parts = d.rest * d.splits, pp = (parts + 7) / 8;
     const int part = idx < pp && xcd * pp + idx < parts ? xcd * pp + idx : -1;
