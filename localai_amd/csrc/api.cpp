@@ -48,9 +48,9 @@ int ensure_device() {
     return LOCALAI_OK;
 }
 
-// The MFMA matvec (gemv_mfma.hip) keeps a second, tile-form copy of Q4_K
-// weights for single-vector decode; LOCALAI_HIP_MFMA_MATVEC=0 turns it off
-// (the row-plane matvec then serves every call).
+// Q4_K, Q6_K and Q8_0 handles hold the tile form that the MFMA kernels read;
+// with LOCALAI_HIP_MFMA_MATVEC=0, read when a handle is made, they hold row
+// planes instead, and the row-plane kernels serve every call on them.
 bool mfma_matvec_enabled() {
     const char *e = getenv("LOCALAI_HIP_MFMA_MATVEC");
     return !(e && e[0] == '0');

@@ -13,14 +13,19 @@
 // 2^-12.
 //
 // Three kernels:
-//   gemm_dense_kernel (gemm_dense.hip) every dense product;
-//   gemm_tile_kernel  the MoE expert tiles on the tile form (Q4_K / Q6_K / Q8_0):
-//                     each wave decodes its own two 16-row tiles into B operands
-//                     in registers, x is staged in LDS (global_load_lds);
-//   gemm_kernel       the MoE expert tiles of types without a tile form (Q4_0,
-//                     Q5_K), from the row planes: a workgroup decodes a 128-row
-//                     weight tile into LDS per 128-value step and 4 waves
-//                     multiply it with 64 tokens.
+//   gemm_dense_kernel (gemm_dense.hip) every dense product of a handle in its
+//                     type's usual form (tile form for Q4_K / Q6_K / Q8_0, row
+//                     planes for Q5_K / Q4_0);
+//   gemm_tile_kernel  the MoE expert tiles on the tile form: each wave decodes
+//                     its own two 16-row tiles into B operands in registers, x
+//                     is staged in LDS (global_load_lds);
+//   gemm_kernel       from the row planes of any type: the MoE expert tiles of
+//                     handles without a tile form (Q4_0, Q5_K, or every type
+//                     with LOCALAI_HIP_MFMA_MATVEC=0), and the dense products of
+//                     Q4_K / Q6_K / Q8_0 handles made with that switch. A
+//                     workgroup decodes a 128-row weight tile into LDS per
+//                     128-value step and 4 waves multiply it with 128 tokens
+//                     (expert tiles: 64).
 #include <type_traits>
 
 #include "gemm_core.h"
@@ -28,6 +33,7 @@
 namespace lq {
 
 constexpr int GM_BM = 128;             // weight rows per workgroup
+constexpr int GM_BN = 128;             // tokens per workgroup (dense)
 constexpr int GM_MOE_BN = 64;          // tokens per workgroup (MoE expert tiles)
 constexpr int GM_LD = GM_BK + 8;       // LDS row stride in halves (272 B: 16 lanes of a
                                        // 16-byte read hit 16 distinct bank groups)
@@ -104,12 +110,12 @@ __global__ __launch_bounds__(256) void x_to_f16_wide_kernel(const float *__restr
 
 // ---------------------------------------------------------------- weights
 
-// Exact fp32 values of unit u in order; the same formulas as
-// engine/dequant.py:62-165.
+// Exact fp32 values of unit u in unit order (the order of gemv_core.h's x
+// windows); the same formulas as engine/dequant.py:62-165. Q8_0 has its own
+// conversion (q8_pairs).
 template <int T>
 __device__ __forceinline__ void dequant_unit(const UnitW &w, int u, float *out) {
-    static_assert(T == LQ_Q5_K || T == LQ_Q4_0, "types without a tile form");
-    if constexpr (T == LQ_Q5_K) {
+    if constexpr (T == LQ_Q4_K || T == LQ_Q5_K) {
         const int p = u & 3;
         uint32_t sc0, sc1, mn0, mn1;
         kq_pair(w.h0, p, sc0, sc1, mn0, mn1);
@@ -119,11 +125,28 @@ __device__ __forceinline__ void dequant_unit(const UnitW &w, int u, float *out) 
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
             const uint32_t byte = (u4_get(j < 16 ? w.q0 : w.q1, (j & 15) >> 2) >> (8 * (j & 3))) & 0xFFu;
-            const uint32_t qh = (u4_get(j < 16 ? w.h1 : w.q2, (j & 15) >> 2) >> (8 * (j & 3))) & 0xFFu;
-            const uint32_t lo = (byte & 15u) | (((qh >> (2 * p)) & 1u) << 4);
-            const uint32_t hi = (byte >> 4) | (((qh >> (2 * p + 1)) & 1u) << 4);
+            uint32_t lo = byte & 15u, hi = byte >> 4;
+            if constexpr (T == LQ_Q5_K) {
+                const uint32_t qh = (u4_get(j < 16 ? w.h1 : w.q2, (j & 15) >> 2) >> (8 * (j & 3))) & 0xFFu;
+                lo |= ((qh >> (2 * p)) & 1u) << 4;
+                hi |= ((qh >> (2 * p + 1)) & 1u) << 4;
+            }
             out[j] = __builtin_fmaf(a0, (float)lo, -b0);
             out[32 + j] = __builtin_fmaf(a1, (float)hi, -b1);
+        }
+    } else if constexpr (T == LQ_Q6_K) {
+        const float d = f16_to_f32(w.d);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float dc = d * (float)(int8_t)(w.sc >> (8 * c));
+            const uint4 ql = (c & 1) ? w.q1 : w.q0;
+            const uint32_t sh = (c >> 1) * 4, hs = 2 * c;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t qb = (u4_get(ql, e >> 2) >> (8 * (e & 3) + sh)) & 15u;
+                const uint32_t hb = (u4_get(w.h0, e >> 2) >> (8 * (e & 3) + hs)) & 3u;
+                out[16 * c + e] = dc * (float)((int)(qb | (hb << 4)) - 32);
+            }
         }
     } else {   // Q4_0
         const float d0 = f16_to_f32(w.sc), d1 = f16_to_f32(w.sc >> 16);
@@ -136,6 +159,13 @@ __device__ __forceinline__ void dequant_unit(const UnitW &w, int u, float *out) 
             out[2 * (j & ~15) + 16 + (j & 15)] = d * (float)((int)(byte >> 4) - 8);
         }
     }
+}
+
+// Position inside the 128-value step window of value j (unit order) of unit u.
+template <int T>
+__device__ __forceinline__ int window_pos(int u, int j) {
+    if constexpr (T == LQ_Q6_K) return 32 * (j >> 4) + 16 * (u & 1) + (j & 15);
+    else return 64 * (u & 1) + j;
 }
 
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
@@ -152,12 +182,32 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 Xs[BN * GM_LD];
     const lq_geom &g = a.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
-    const int64_t rtile = blockIdx.x;
-    const int tile = blockIdx.y;
-    if (tile >= a.n_tiles[0]) return;
-    const uint8_t *W = a.W + (int64_t)a.tile_e[tile] * g.matrix_bytes;
-    const int64_t p0 = a.tile_p0[tile];
-    const int tn = a.tile_n[tile];
+    // token tile
+    const uint8_t *W = a.W;
+    int64_t p0;
+    int tn;
+    int64_t rtile;
+    if constexpr (MODE == GM_DENSE) {
+        // 1-D grid, padded to a multiple of 8. Workgroups are dispatched to the
+        // 8 XCDs round-robin (id % 8); workgroup id -> logical index
+        // xcd * per + id / 8 walks the row tiles of one token tile per XCD, so
+        // each XCD's L2 holds one activation tile while the weights stream.
+        const int id = blockIdx.x, per = gridDim.x / 8;
+        const int L = (id % 8) * per + id / 8;
+        const int nrt = (int)((g.rows + GM_BM - 1) / GM_BM);
+        const int64_t ntt = (a.ntok + BN - 1) / BN;
+        if (L >= nrt * ntt) return;
+        rtile = L % nrt;
+        p0 = (int64_t)(L / nrt) * BN;
+        tn = (int)(a.ntok - p0 < BN ? a.ntok - p0 : BN);
+    } else {
+        rtile = blockIdx.x;
+        const int tile = blockIdx.y;
+        if (tile >= a.n_tiles[0]) return;
+        W += (int64_t)a.tile_e[tile] * g.matrix_bytes;
+        p0 = a.tile_p0[tile];
+        tn = a.tile_n[tile];
+    }
     // weight rows of this tile: q -> matrix row (or -1 when past the end)
     const int64_t r0 = rtile * (MODE == GM_MOE_GATE_UP ? GM_BM / 2 : GM_BM);
     auto row_of = [&](int q) -> int64_t {
@@ -198,16 +248,32 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
         const int u = 2 * step + lh;
         const bool valid = u < U;
         _Float16 *wd = Ws + lr * GM_LD;
-        float v[64];
-        dequant_unit<T>(wreg, u < U ? u : U - 1, v);
+        if constexpr (T == LQ_Q8_0) {
+            const uint32_t dm = valid ? 0xFFFFFFFFu : 0u;
+            const lq_h2 d0 = __builtin_bit_cast(lq_h2, ((wreg.sc & 0xFFFFu) * 0x10001u) & dm);
+            const lq_h2 d1 = __builtin_bit_cast(lq_h2, ((wreg.sc >> 16) * 0x10001u) & dm);
+            const uint4 qs[4] = {wreg.q0, wreg.q1, wreg.q2, wreg.q3};
 #pragma unroll
-        for (int j = 0; j < 64; j += 8) {
-            uint4 p;
-            p.x = valid ? pack_h2(v[j + 0], v[j + 1]) : 0u;
-            p.y = valid ? pack_h2(v[j + 2], v[j + 3]) : 0u;
-            p.z = valid ? pack_h2(v[j + 4], v[j + 5]) : 0u;
-            p.w = valid ? pack_h2(v[j + 6], v[j + 7]) : 0u;
-            *reinterpret_cast<uint4 *>(wd + 64 * (u & 1) + j) = p;
+            for (int c = 0; c < 8; ++c) {      // 8 values per 16-byte LDS write
+                const uint4 q = qs[c >> 1];
+                const lq_h2 d2 = c < 4 ? d0 : d1;
+                uint4 p;
+                q8_pairs(u4_get(q, 2 * (c & 1)), d2, p.x, p.y);
+                q8_pairs(u4_get(q, 2 * (c & 1) + 1), d2, p.z, p.w);
+                *reinterpret_cast<uint4 *>(wd + 64 * (u & 1) + 8 * c) = p;
+            }
+        } else {
+            float v[64];
+            dequant_unit<T>(wreg, u < U ? u : U - 1, v);
+#pragma unroll
+            for (int j = 0; j < 64; j += 8) {
+                uint4 p;
+                p.x = valid ? pack_h2(v[j + 0], v[j + 1]) : 0u;
+                p.y = valid ? pack_h2(v[j + 2], v[j + 3]) : 0u;
+                p.z = valid ? pack_h2(v[j + 4], v[j + 5]) : 0u;
+                p.w = valid ? pack_h2(v[j + 6], v[j + 7]) : 0u;
+                *reinterpret_cast<uint4 *>(wd + window_pos<T>(u, j)) = p;
+            }
         }
         uint4 *xd = reinterpret_cast<uint4 *>(Xs + xr * GM_LD + XV * xp);
 #pragma unroll
@@ -655,9 +721,9 @@ template <int MODE, int BN>
 static int launch_gemm_t(const GemmArgs &a, dim3 grid, hipStream_t s) {
     switch (a.g.type) {
 #define LQ_GM(TT) case TT: hipLaunchKernelGGL((gemm_kernel<TT, BN, MODE>), grid, dim3(256), 0, s, a); break;
-        LQ_GM(LQ_Q5_K) LQ_GM(LQ_Q4_0)
+        LQ_GM(LQ_Q4_K) LQ_GM(LQ_Q5_K) LQ_GM(LQ_Q6_K) LQ_GM(LQ_Q8_0) LQ_GM(LQ_Q4_0)
 #undef LQ_GM
-        default: return fail(LOCALAI_ETYPE, "moe: unsupported expert type");
+        default: return fail(LOCALAI_ETYPE, "matmul: unsupported GGML type");
     }
     LQ_HIP(hipGetLastError());
     return LOCALAI_OK;
@@ -685,8 +751,14 @@ int launch_gemm(const lq_geom &g, const uint8_t *W, const uint8_t *Wt, const flo
     GemmArgs a{};
     a.g = g; a.W = W; a.Xh = Xh; a.ldh = (int)ldh; a.inv = inv; a.ntok = ntok; a.Y = Y; a.y_ts = y_ts; a.y_rs = y_rs;
     a.Wt = Wt;
-    const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
+    // a type with a tile form, in a handle made without one (mfma_matvec_enabled)
+    const bool planes = !Wt && mt_matrix_bytes(g) > 0;
+    const int64_t nwg = ((g.rows + GM_BM - 1) / GM_BM) * ((ntok + GM_BN - 1) / GM_BN);
+    if (!Wt && !W) return fail(LOCALAI_ESTATE, "matmul: handle without weights");
+    if (planes && nwg > ((int64_t)1 << 30)) return fail(LOCALAI_EARG, "matmul: problem too large");
     if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
+    if (planes) return launch_gemm_t<GM_DENSE, GM_BN>(a, dim3((unsigned)((nwg + 7) / 8 * 8)), s);
+    const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
     return launch_gemm_dense(a, (uint8_t *)ws + xb, ws_bytes > xb ? ws_bytes - xb : 0, s);
 }
 
@@ -718,6 +790,7 @@ int launch_moe_gemm(const lq_geom &g, const uint8_t *Wall, const uint8_t *Wt_all
         return launch_gemm_tile_t<GM_MOE_DOWN, GM_MOE_BN, NW>(
             a, dim3((unsigned)((g.rows + 32 * NW - 1) / (32 * NW)), (unsigned)max_tiles), s);
     }
+    if (!Wall) return fail(LOCALAI_ESTATE, "moe: expert handle without row planes");
     if (gate_up) {
         dim3 grid((unsigned)((inter + GM_BM / 2 - 1) / (GM_BM / 2)), (unsigned)max_tiles);
         return launch_gemm_t<GM_MOE_GATE_UP, GM_MOE_BN>(a, grid, s);

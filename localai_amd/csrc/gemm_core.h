@@ -38,7 +38,7 @@ __device__ __forceinline__ void q8_pairs(uint32_t w, lq_h2 d2, uint32_t &lo, uin
     hi = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(lq_h2, h) - off) * d2);
 }
 
-enum { GM_MOE_GATE_UP = 1, GM_MOE_DOWN = 2 };
+enum { GM_DENSE = 0, GM_MOE_GATE_UP = 1, GM_MOE_DOWN = 2 };
 
 // Dense: Xh [ntok, ldh]; Y[t * y_ts + r * y_rs].
 // MoE: work tile blockIdx.y of the expert tile list (expert, first row of

@@ -705,6 +705,9 @@ int64_t gemm_dense_split_bytes(const lq_geom &g, int64_t ntok) { return ntok < 1
 int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hipStream_t s) {
     constexpr int lds = GD_RING * GD_SLOT;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
+    // the kernel is chosen by type alone: its weights must be the ones it reads
+    if (a.g.type == LQ_Q5_K || a.g.type == LQ_Q4_0 ? !a.W : !a.Wt)
+        return fail(LOCALAI_ESTATE, "matmul: handle without the weights' form");
     DensePlan p = dense_plan(a.g, a.ntok);
     if (p.rest) p.fit(gd_blocks(a.g), split_bytes / (p.rest * GD_PART * 4));
     // 32-bit byte offsets into the 128 x rows of a workgroup

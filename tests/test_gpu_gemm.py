@@ -9,6 +9,8 @@ accumulation adds K * 2^-24 of the same sum). Gates: every output within
 the sum cancels), and the path's max-rel 1e-3 target (normwise:
 max|y - y_ref| / max|y_ref|) for tiles of at least 64 outputs, where the
 typical figure is near 2e-4."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -134,6 +136,37 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     got = gpu_matmul(raw, t, rows, cols, xs)
     check(got, raw, t, rows, cols, xs)
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
+
+
+@pytest.mark.parametrize('t', (12, 14, 8))
+@pytest.mark.parametrize('rows,cols,tokens', [(300, 512, 130), (129, 1280, 33), (16, 768, 7), (200, 160, 257)])
+def test_handles_without_the_tile_form(monkeypatch, t, rows, cols, tokens):
+    """LOCALAI_HIP_MFMA_MATVEC=0 when a handle is made: Q4_K, Q6_K and Q8_0 hold
+    row planes, and their products, in both layouts, through the handle and
+    through the legacy export, come from those."""
+    from localai_amd import _lib, device
+    if cols % quant.block_layout(t)[0]:
+        cols += 256 - cols % 256
+    rng = np.random.default_rng(rows + cols + t)
+    raw = random_ggml(rng, t, rows * cols)
+    xs = rng.standard_normal((tokens, cols)).astype(np.float32)
+    monkeypatch.setenv('LOCALAI_HIP_MFMA_MATVEC', '0')
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    xd = device.to_device_f32(xs)
+    got = q.matmul(xd).cpu().numpy()
+    check(got, raw, t, rows, cols, xs)
+    np.testing.assert_array_equal(q.matmul(xd, rows_major=True).cpu().numpy(), got.T)
+    assert normwise_rel(q.matvec(xd[0].contiguous()).cpu().numpy(), quant.matmul_exact(raw, t, rows, cols, xs[:1])[0]) < 1e-5
+    q.close()
+    lib = _lib.load()
+    out = np.zeros((rows, tokens), np.float32)
+    buf = np.frombuffer(raw, np.uint8)
+    f32 = ctypes.POINTER(ctypes.c_float)
+    getattr(lib, {12: 'localai_q4k_matmul', 14: 'localai_q6k_matmul', 8: 'localai_q8_0_matmul'}[t])(
+        buf.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8)), xs.ctypes.data_as(f32), out.ctypes.data_as(f32), rows,
+        cols, tokens, 4)
+    assert lib.localai_hip_last_status() == 0
+    check(out.T, raw, t, rows, cols, xs)
 
 
 @pytest.mark.parametrize('t', (2, 8))

@@ -98,6 +98,23 @@ def test_gemm_path_threshold_and_ragged_tiles(t, T):
     assert normwise_rel(out, rout) < (1e-5 if T < 32 else 1e-3)
 
 
+@pytest.mark.parametrize('t,I', [(12, 256), (14, 256), (8, 320)])
+@pytest.mark.parametrize('T', (2, 67))
+def test_experts_without_the_tile_form(monkeypatch, t, I, T):
+    """LOCALAI_HIP_MFMA_MATVEC=0 when the expert handles are made: decode and
+    prefill run from their row planes."""
+    from localai_amd import synth
+    monkeypatch.setenv('LOCALAI_HIP_MFMA_MATVEC', '0')
+    rng = np.random.default_rng(T * 5 + t)
+    E, H, k = 8, 512, 2
+    rw, gu, dn = make_layer(rng, E, H, I, t)
+    h = synth.activations(rng, T, H)
+    (out, idx, g), (rout, ridx, rg) = run_both(rw, gu, dn, t, E, H, I, k, h)
+    np.testing.assert_array_equal(idx, ridx)
+    np.testing.assert_allclose(g, rg, rtol=1e-5, atol=1e-6)
+    assert normwise_rel(out, rout) < (1e-5 if T < 32 else 1e-3)
+
+
 def test_forced_router_ties_pick_lower_index():
     from localai_amd import synth
     rng = np.random.default_rng(8)
