@@ -235,7 +235,7 @@ __device__ __forceinline__ void gd_dma(const void *base, uint32_t off, uint32_t 
 // computed whole, one per workgroup and round; the rest .. are cut `splits` ways
 // in K, part i covering blocks [i * blocks, ...). With splits > 1 the parts go to
 // P, part i of rest tile k at P + (i * rest + k) * GD_PART, in Y's order (rows or
-// tokens fastest), and gemm_split_sum_kernel adds them.
+// tokens fastest) and not yet scaled, and gemm_split_sum_kernel adds them.
 struct DenseArgs {
     GemmArgs a;
     int full, rest, splits, blocks;
@@ -506,8 +506,9 @@ struct GdMain {
     }
     // D: the lane holds token lane % 16 of token tile i and rows 4 (lane / 16) +
     // v of row tile j: one 16-byte store where rows are contiguous. out points
-    // at the tile's first row and token
-    __device__ __forceinline__ void store(const GemmArgs &a, int rb, int tt, float *out, int64_t ts, int64_t rs) {
+    // at the tile's first row and token; scaled: results, else a part's sums
+    __device__ __forceinline__ void store(const GemmArgs &a, int rb, int tt, float *out, int64_t ts, int64_t rs,
+                                          bool scaled) {
         fresh_lane();
         const int fr = lane & 15, q = lane >> 4;
         const int64_t p0 = (int64_t)tt * GD_BN, r0 = (int64_t)rb * GD_BM;
@@ -518,7 +519,7 @@ struct GdMain {
         for (int i = 0; i < NV; ++i) {
             const int lt = 16 * i + fr;
             if (lt >= tn) continue;
-            const float sc = a.inv[p0 + lt];
+            const float sc = scaled ? a.inv[p0 + lt] : 1.0f;
             float *yp = out + lt * ts;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -588,10 +589,11 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
                 start();
             }
             if (to_y)
-                m.store(a, rb0, tt0, a.Y + (int64_t)tt0 * GD_BN * a.y_ts + (int64_t)rb0 * GD_BM * a.y_rs, a.y_ts, a.y_rs);
+                m.store(a, rb0, tt0, a.Y + (int64_t)tt0 * GD_BN * a.y_ts + (int64_t)rb0 * GD_BM * a.y_rs, a.y_ts, a.y_rs,
+                        true);
             else
                 m.store(a, rb0, tt0, d.P + ((int64_t)sp0 * d.rest + (tile0 - d.full)) * GD_PART,
-                        a.y_rs == 1 ? GD_BM : 1, a.y_rs == 1 ? 1 : GD_BN);
+                        a.y_rs == 1 ? GD_BM : 1, a.y_rs == 1 ? 1 : GD_BN, false);
             if (!more) break;
         }
     };
@@ -611,8 +613,10 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void gemm_dense_kernel(DenseArgs d) 
     }
 }
 
-// Y of the rest tiles = the sum of their parts, in part order (workgroup: tile
-// blockIdx.x, 16 of its 128 tokens or 32 of its 256 rows, whichever runs slowest)
+// Y of the rest tiles = the sum of their parts, in part order, times the token's
+// scale (a power of two; the parts are unscaled, in the range of f16 products:
+// scaled ones could overflow where the whole does not). Workgroup: tile
+// blockIdx.x, 16 of its 128 tokens or 32 of its 256 rows, whichever runs slowest
 __global__ __launch_bounds__(256) void gemm_split_sum_kernel(DenseArgs d) {
     const GemmArgs &a = d.a;
     const int ntt = (int)((a.ntok + GD_BN - 1) / GD_BN), nrb = (int)((a.g.rows + GD_BM - 1) / GD_BM);
@@ -633,7 +637,12 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(DenseArgs d) {
     for (int h = 0; h < 4; ++h) {
         const int e = (int)blockIdx.y * 4096 + 1024 * h + 4 * (int)threadIdx.x, si = e / nfast, fi = e % nfast;
         if (si >= sn || fi >= fn) continue;
-        lq_f4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        lq_f4 sc, sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int tk = rows_fast ? si : fi + k;
+            sc[k] = a.inv[p0 + (tk < tn ? tk : tn - 1)];
+        }
         for (int k0 = 0; k0 < d.splits; k0 += 8) {
             lq_f4 v[8];
 #pragma unroll
@@ -643,6 +652,7 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(DenseArgs d) {
             for (int k = 0; k < 8; ++k)
                 if (k0 + k < d.splits) sum += v[k];
         }
+        sum *= sc;
         float *y = Y + si * ys + fi;
         if (vec && fi + 3 < fn) {
             *reinterpret_cast<lq_f4 *>(y) = sum;

@@ -138,6 +138,42 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
 
 
+@pytest.mark.parametrize('t', TYPES)
+@pytest.mark.parametrize('rows_major', (False, True))
+def test_parts_of_huge_activations_cancel(t, rows_major):
+    """Rows of x near fp32's largest values whose halves cancel in the product:
+    each half's sum exceeds fp32, the whole does not, however K is divided.
+    One positive weight throughout (its type's bytes), so every output of a
+    token is the sum of its x times that weight."""
+    from localai_amd import device
+    rows, cols, tokens = 300, 4096, 33
+    block, size = quant.block_layout(t)
+    b = np.zeros((rows * cols // block, size), np.uint8)
+    d = 208 if t == 14 else 0
+    b[:, d:d + 2] = np.frombuffer(np.float16(0.002).tobytes(), np.uint8)
+    if t in (12, 13):
+        b[:, 4:12], b[:, 12:16] = 1, 0x11   # scales 1 (of dmin, which is 0, too)
+        b[:, 16:48] = 0x11 if t == 12 else 0
+        b[:, 48:] = 0x11                    # quants 1
+    elif t == 14:
+        b[:, 128:192], b[:, 192:208] = 0xAA, 1   # high bits 2: quants 32 - 32 + 1
+        b[:, :128] = 0x11
+    else:
+        b[:, 2:] = 1 if t == 8 else 0x99    # quants 1 (Q4_0: 9 - 8)
+    raw = b.tobytes()
+    w = quant.dequantize(raw, t, (rows, cols)).astype(np.float64)
+    assert w.min() == w.max() > 0.0019
+    # exact in f16: with values that are not, the rounding of each half (up to
+    # 2^-11 of it) would be 15 times that of the whole in normwise_rel
+    xs = np.full((tokens, cols), 2.0 ** 127, np.float32)
+    xs[:, cols // 2:] *= np.float32(-0.875)
+    xs[1] = 1.0
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    got = q.matmul(device.to_device_f32(xs), rows_major=rows_major).cpu().numpy()
+    q.close()
+    check(got.T if rows_major else got, raw, t, rows, cols, xs)
+
+
 @pytest.mark.parametrize('t', (12, 14, 8))
 @pytest.mark.parametrize('rows,cols,tokens', [(300, 512, 130), (129, 1280, 33), (16, 768, 7), (200, 160, 257)])
 def test_handles_without_the_tile_form(monkeypatch, t, rows, cols, tokens):
