@@ -683,7 +683,8 @@ int launch_x_to_f16(const float *X, int64_t ldx, int64_t cols, const int32_t *ro
     if (cols % 8 || ldh % 8 || ldh < cols) return fail(LOCALAI_EARG, "f16 rows: cols % 8 != 0");
     const int vec = (uintptr_t)X % 16 == 0 && ldx % 4 == 0;
     const int per = (int)((ldh / 8 + 63) / 64);   // 8-value groups per lane
-    if (per > 4 && per <= 32 && !nrm2) {
+    // (a launch has fewer than 2^32 threads)
+    if (per > 4 && per <= 32 && !nrm2 && ntok < ((int64_t)1 << 24)) {
         auto gw = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3((unsigned)ntok), dim3(256), 0, s, X, ldx, (int)cols, rows_map, k, Xh,
                                (int)ldh, inv, vec);
@@ -751,15 +752,28 @@ int launch_gemm(const lq_geom &g, const uint8_t *W, const uint8_t *Wt, const flo
     GemmArgs a{};
     a.g = g; a.W = W; a.Xh = Xh; a.ldh = (int)ldh; a.inv = inv; a.ntok = ntok; a.Y = Y; a.y_ts = y_ts; a.y_rs = y_rs;
     a.Wt = Wt;
-    // a type with a tile form, in a handle made without one (mfma_matvec_enabled)
-    const bool planes = !Wt && mt_matrix_bytes(g) > 0;
+    // row planes of a type with a tile form (a handle made without one,
+    // mfma_matvec_enabled), or with rows past the dense kernel's 32-bit offsets
+    // into 16 of them
+    const bool planes = !Wt && (mt_matrix_bytes(g) > 0 || g.cols >= ((int64_t)1 << 29));
     const int64_t nwg = ((g.rows + GM_BM - 1) / GM_BM) * ((ntok + GM_BN - 1) / GM_BN);
     if (!Wt && !W) return fail(LOCALAI_ESTATE, "matmul: handle without weights");
-    if (planes && nwg > ((int64_t)1 << 30)) return fail(LOCALAI_EARG, "matmul: problem too large");
+    // tokens per launch: the dense kernel's 32-bit byte offsets into a tile's x rows
+    const int64_t most = planes ? ntok : (((int64_t)1 << 32) - 1) / (2 * ldh);
+    if (most < 1 || (planes && nwg > ((int64_t)1 << 30))) return fail(LOCALAI_EARG, "matmul: problem too large");
     if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
     if (planes) return launch_gemm_t<GM_DENSE, GM_BN>(a, dim3((unsigned)((nwg + 7) / 8 * 8)), s);
     const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
-    return launch_gemm_dense(a, (uint8_t *)ws + xb, ws_bytes > xb ? ws_bytes - xb : 0, s);
+    for (int64_t t0 = 0; t0 < ntok;) {
+        // (a tile has 128 tokens: all in one launch below 16.7 million columns)
+        a.ntok = most < GM_BN && ntok - t0 > most ? most : ntok - t0;
+        a.Xh = Xh + t0 * ldh;
+        a.inv = inv + t0;
+        a.Y = Y + t0 * y_ts;
+        if (int st = launch_gemm_dense(a, (uint8_t *)ws + xb, ws_bytes > xb ? ws_bytes - xb : 0, s)) return st;
+        t0 += a.ntok;
+    }
+    return LOCALAI_OK;
 }
 
 int moe_gemm_tile() { return GM_MOE_BN; }

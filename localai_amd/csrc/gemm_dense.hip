@@ -269,8 +269,8 @@ struct GdMain {
     // row planes: first row of each row tile in each plane, the lane's row in
     // the tile, units of a row, the split's first block
     const uint8_t *pl[2][3];
-    int dr[2], nu, first;
-    int pitch[3];
+    int nu, first;
+    uint32_t dr[2], pitch[3];
     float sa[2], sm[2];            // Q5_K: scale and minimum of the slices' sub-block
     const uint8_t *xb;             // x row p0 at the split's first value
     uint32_t xoff[XN];
@@ -302,8 +302,8 @@ struct GdMain {
             const int off = 16 * (du + (c & 1) * C);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                cu_load(d[j].q, pl[j][0] + 16 * (c0 + (int64_t)u), (uint32_t)(dr[j] * pitch[0] + off));
-                if constexpr (T == LQ_Q4_0) cu_load(d[j].d, pl[j][1] + 4 * (int64_t)u, (uint32_t)(dr[j] * pitch[1] + 4 * du));
+                cu_load(d[j].q, pl[j][0] + 16 * (c0 + (int64_t)u), dr[j] * pitch[0] + (uint32_t)off);
+                if constexpr (T == LQ_Q4_0) cu_load(d[j].d, pl[j][1] + 4 * (int64_t)u, dr[j] * pitch[1] + (uint32_t)(4 * du));
             }
             return;
         } else {
@@ -319,8 +319,8 @@ struct GdMain {
             const int off = 16 * ((lane >> 4) & 1) * (nsb - s0 < 16 ? nsb - s0 : 16);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                cu_load(d[j].qh, pl[j][1] + 16 * (s0 + (int64_t)sb), (uint32_t)(dr[j] * pitch[1] + off));
-                cu_load(d[j].h, pl[j][2] + 16 * (int64_t)sb, (uint32_t)(dr[j] * pitch[2]));
+                cu_load(d[j].qh, pl[j][1] + 16 * (s0 + (int64_t)sb), dr[j] * pitch[1] + (uint32_t)off);
+                cu_load(d[j].h, pl[j][2] + 16 * (int64_t)sb, dr[j] * pitch[2]);
             }
         } else {
             const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
@@ -481,11 +481,11 @@ struct GdMain {
             first = (int)sb0;
             nu = (int)a.g.nu;
 #pragma unroll
-            for (int p = 0; p < 3; ++p) pitch[p] = (int)a.g.pitch[p];
+            for (int p = 0; p < 3; ++p) pitch[p] = (uint32_t)a.g.pitch[p];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int64_t r = (t0 + j < tiles ? t0 + j : tiles - 1) * MT_ROWS;
-                dr[j] = (int)(r + (lane & 15) < a.g.rows ? lane & 15 : a.g.rows - 1 - r);
+                dr[j] = (uint32_t)(r + (lane & 15) < a.g.rows ? lane & 15 : a.g.rows - 1 - r);
 #pragma unroll
                 for (int p = 0; p < 3; ++p) pl[j][p] = a.W + a.g.plane[p] + r * a.g.pitch[p];
             }
@@ -501,7 +501,7 @@ struct GdMain {
 #pragma unroll
         for (int i = 0; i < XN; ++i) {
             const int row = (GD_NW * i + wave) * 4 + (lane >> 4), c = (lane & 15) ^ (row & 15);
-            xoff[i] = (uint32_t)((row < tn ? row : 0) * a.ldh * 2 + 16 * c);
+            xoff[i] = (uint32_t)(row < tn ? row : 0) * (uint32_t)a.ldh * 2u + 16u * (uint32_t)c;
         }
     }
     // D: the lane holds token lane % 16 of token tile i and rows 4 (lane / 16) +
@@ -720,8 +720,8 @@ int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hi
         return fail(LOCALAI_ESTATE, "matmul: handle without the weights' form");
     DensePlan p = dense_plan(a.g, a.ntok);
     if (p.rest) p.fit(gd_blocks(a.g), split_bytes / (p.rest * GD_PART * 4));
-    // 32-bit byte offsets into the 128 x rows of a workgroup
-    if ((int64_t)a.ldh * 2 * GD_BN >= ((int64_t)1 << 32) || p.tiles > ((int64_t)1 << 30))
+    // 32-bit byte offsets into the x rows of a workgroup
+    if ((int64_t)a.ldh * 2 * (a.ntok < GD_BN ? a.ntok : GD_BN) >= ((int64_t)1 << 32) || p.tiles > ((int64_t)1 << 30))
         return fail(LOCALAI_EARG, "matmul: problem too large");
     const DenseArgs d{a, p.full, p.rest, p.splits, p.blocks, (float *)split_ws};
     const dim3 grid(p.full ? 256 : (unsigned)((p.rest * p.splits + 7) / 8 * 8));

@@ -138,6 +138,38 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
 
 
+@pytest.mark.parametrize('t,rows,cols,tokens', [(2, 3, (1 << 25) + 32, 66), (8, 3, (1 << 25) + 32, 66),
+                                                (2, 1, (1 << 28) + 32, 1)])
+def test_rows_past_32_bit_offsets(t, rows, cols, tokens):
+    """More than 4 GiB of f16 rows of x under one token tile (33.6 million columns,
+    66 tokens): several launches, each with offsets of 32 bits, the same products
+    in both layouts; and a row of 268 million columns. x holds zeros but for
+    2^16 values (the row's ends among them), so that fp32 sums over millions of
+    products stay exact enough to compare."""
+    from localai_amd import device
+    torch = device.torch()
+    rng = np.random.default_rng(t)
+    block, size = quant.block_layout(t)
+    part = np.frombuffer(random_ggml(rng, t, 1 << 20), np.uint8).reshape(-1, size)
+    raw = np.resize(part, (rows * cols // block, size)).tobytes()
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    at = np.unique(np.concatenate([rng.integers(0, cols, 1 << 16), np.arange(64), np.arange(cols - 64, cols)]))
+    vals = device.to_device_f32(rng.standard_normal((tokens, len(at))))
+    at = torch.from_numpy(at).to(vals.device)
+    x = torch.zeros((tokens, cols), dtype=torch.float32, device=vals.device)
+    x[:, at] = vals
+    got = q.matmul(x)
+    assert torch.equal(q.matmul(x, rows_major=True), got.T)
+    w = q.dequant()[:, at].double()
+    for tok in range(tokens):
+        terms = w * vals[tok].double()
+        # products of random sign, x and w each rounded by up to 2^-11 of them,
+        # evenly: five standard deviations of their sum
+        bound = 5 * 2.0 ** -11 * (2 / 3) ** 0.5 * terms.square().sum(1).sqrt()
+        assert bool((got[tok].double() - terms.sum(1)).abs().le(bound).all())
+    q.close()
+
+
 @pytest.mark.parametrize('t', TYPES)
 @pytest.mark.parametrize('rows_major', (False, True))
 def test_parts_of_huge_activations_cancel(t, rows_major):
