@@ -13,12 +13,13 @@
 // 2^-12.
 //
 // Three kernels:
-//   gemm_dense_kernel (gemm_dense.hip) every dense product of a handle in its
+//   gemm_dense_kernel (gemm_dense.hip) dense products of handles in their
 //                     type's usual form (tile form for Q4_K / Q6_K / Q8_0, row
 //                     planes for Q5_K / Q4_0);
-//   gemm_tile_kernel  the MoE expert tiles on the tile form: each wave decodes
-//                     its own two 16-row tiles into B operands in registers, x
-//                     is staged in LDS (global_load_lds);
+//   gemm_tile_kernel  the MoE expert tiles and the dense products of short K
+//                     (gemm_takes_tile_kernel) on the tile form: each wave
+//                     decodes its own two 16-row tiles into B operands in
+//                     registers, x is staged in LDS (global_load_lds);
 //   gemm_kernel       from the row planes of any type: the MoE expert tiles of
 //                     handles without a tile form (Q4_0, Q5_K, or every type
 //                     with LOCALAI_HIP_MFMA_MATVEC=0), and the dense products of
@@ -350,7 +351,8 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 // through LDS, double-buffered and shared by the waves.
 //
 // Workgroup: 8 waves x 2 row tiles (256 weight rows; for gate_up 128 gate rows
-// and the 128 matching up rows) x 64 tokens, 128 K values per step.
+// and the 128 matching up rows) x 64 tokens; dense: 4 waves x 2 row tiles x 128
+// tokens; 128 K values per step.
 
 constexpr int GM_MOE_NW = 8;           // waves per workgroup of the expert tile GEMMs
 
@@ -619,7 +621,8 @@ __device__ __forceinline__ void gt_main(const GemmArgs &a, _Float16 (*Xs)[BN * G
 
 // NW waves per workgroup (4 or 8): 32 NW weight rows (gate_up: 16 NW gate and
 // 16 NW up rows) share one staged x tile; 8 waves halve the x bytes each
-// weight byte brings along (the MoE expert tiles)
+// weight byte brings along (the MoE expert tiles);
+// dense products of short K run 4
 template <int T, int BN, int MODE, int NW = 4>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) {
     constexpr int NI = BN / 16;            // 16-token MFMA tiles per wave
@@ -631,16 +634,33 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) 
     // wave index made wave-uniform: row-tile addresses go to scalar registers
     // (MoE Q4_K GEMMs 162 -> 128 VGPRs; gate_up 85 -> 81 us, down 55 -> 48 us)
     const int wave = wave_id();
-    const int64_t blk = blockIdx.x;
-    const int tile = blockIdx.y;
-    if (tile >= a.n_tiles[0]) return;
-    const uint8_t *Wt = a.Wt + (int64_t)a.tile_e[tile] * a.wt_bytes;
-    // the expert's row norms (gate_up with f16 output)
-    const float *wn = a.wnorm ? a.wnorm + 2 * (int64_t)a.tile_e[tile] : nullptr;
-    const int64_t p0 = a.tile_p0[tile];
-    const int tn = a.tile_n[tile];
+    const uint8_t *Wt = a.Wt;
+    int64_t p0;
+    int tn;
+    int64_t blk;
+    const float *wn = nullptr;   // the expert's row norms (gate_up with f16 output)
+    if constexpr (MODE == GM_DENSE) {
+        // 1-D grid, padded to a multiple of 8; workgroup id -> logical index
+        // xcd * per + id / 8 walks the row blocks of one token tile per XCD
+        const int id = blockIdx.x, per = gridDim.x / 8;
+        const int L = (id % 8) * per + id / 8;
+        const int nrb = (int)((g.rows + 32 * NW - 1) / (32 * NW));
+        const int64_t ntt = (a.ntok + BN - 1) / BN;
+        if (L >= nrb * ntt) return;
+        blk = L % nrb;
+        p0 = (int64_t)(L / nrb) * BN;
+        tn = (int)(a.ntok - p0 < BN ? a.ntok - p0 : BN);
+    } else {
+        blk = blockIdx.x;
+        const int tile = blockIdx.y;
+        if (tile >= a.n_tiles[0]) return;
+        Wt += (int64_t)a.tile_e[tile] * a.wt_bytes;
+        if (a.wnorm) wn = a.wnorm + 2 * (int64_t)a.tile_e[tile];
+        p0 = a.tile_p0[tile];
+        tn = a.tile_n[tile];
+    }
     const int64_t tiles = (g.rows + MT_ROWS - 1) / MT_ROWS, nsb = mt_nsb(g);
-    // the wave's two row tiles: down 2 NW blk + 2 wave + j; gate_up
+    // the wave's two row tiles: dense / down 2 NW blk + 2 wave + j; gate_up
     // gate tile NW blk + wave (j = 0) and its up tile inter / 16 + NW blk + wave
     int64_t t0, t1;
     if constexpr (MODE == GM_MOE_GATE_UP) {
@@ -652,13 +672,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) 
     }
     const uint8_t *w0p = Wt + (t0 < tiles ? t0 : tiles - 1) * nsb * BB;
     const uint8_t *w1p = Wt + (t1 < tiles ? t1 : tiles - 1) * nsb * BB;
-    // one copy of the loop per count of 16-token tiles
-    static_assert(BN == 64, "up to four 16-token tiles");
-    const int nv = __builtin_amdgcn_readfirstlane((tn + 15) >> 4);
-    if (nv == 1) gt_main<T, BN, MODE, NW, 1>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-    else if (nv == 2) gt_main<T, BN, MODE, NW, 2>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-    else if (nv == 3) gt_main<T, BN, MODE, NW, 3>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
-    else gt_main<T, BN, MODE, NW, 4>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    if constexpr (MODE == GM_DENSE) {
+        gt_main<T, BN, MODE, NW, NI>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    } else {
+        // expert tiles: one copy of the loop per count of 16-token tiles
+        static_assert(NI == 4, "up to four 16-token tiles");
+        const int nv = __builtin_amdgcn_readfirstlane((tn + 15) >> 4);
+        if (nv == 1) gt_main<T, BN, MODE, NW, 1>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+        else if (nv == 2) gt_main<T, BN, MODE, NW, 2>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+        else if (nv == 3) gt_main<T, BN, MODE, NW, 3>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+        else gt_main<T, BN, MODE, NW, 4>(a, Xs, tsc, asc, wn, w0p, w1p, p0, tn, t0, t1, tiles, nsb);
+    }
 }
 
 // ---------------------------------------------------------------- host side
@@ -672,8 +696,41 @@ static int64_t gemm_x_bytes(const lq_geom &g, int64_t ntok) {
     return lq_align256((ntok + 15) / 16 * 16 * gemm_ldh(g) * 2) + ntok * 4;
 }
 
+// Whether a dense product on the tile form runs gemm_tile_kernel (128 x 128 tiles,
+// two workgroups per CU) instead of gemm_dense_kernel (256 x 128, one, K divided).
+// Where K is short, the dense kernel's first loads, its larger stores and the sum
+// of its parts take longer than the blocks: the smaller tiles then win as long as
+// their workgroups come to about one per CU. Both times from fits over whole
+// calls (gemm_dense_us; the tile kernel's: 0.95 to 1.05 of the measured in 98 of
+// 100 calls). 2048 x 768, 512 tokens: Q4_K 20.5 us dense, 16.5 here, Q6_K 21.5,
+// 17.1; 1024 x 1024, 700 tokens Q4_K 24.1, 19.4; 11008 x 2048, 256 tokens 34.8,
+// 30.7; but 4096 x 4096, 128 tokens 26.9, 50.3 and 11008 x 2048, 300 tokens 34.5,
+// 39.0. Of 5160 calls up to 32000 rows the choice is within 4 % of the faster
+// kernel in all but 80, at worst 13 % off (11 % where it stays with the dense one).
+// Up to 32 tokens the dense kernel computes a quarter of what this one does.
+// (The tile kernel's offsets into Y have 32 bits.)
+// *split_bytes: what the parts of K of the dense kernel take, 0 with the tile kernel.
+static bool gemm_takes_tile_kernel(const lq_geom &g, int64_t ntok, int64_t *split_bytes) {
+    const double dense = gemm_dense_us(g, ntok, split_bytes);
+    if (mt_matrix_bytes(g) == 0 || ntok <= 32 || g.rows >= ((int64_t)1 << 25)) return false;
+    const int64_t nwg = ((g.rows + GM_BM - 1) / GM_BM) * ((ntok + GM_BN - 1) / GM_BN), left = nwg % 512;
+    // us per block: a full round of 512 workgroups, one of up to 256, of more
+    const double full = g.type == LQ_Q4_K ? 3.75 : g.type == LQ_Q6_K ? 4.15 : 3.9;
+    const double half = g.type == LQ_Q4_K ? 2.6 : g.type == LQ_Q6_K ? 2.7 : 2.4;
+    const double most = g.type == LQ_Q4_K ? 3.55 : g.type == LQ_Q6_K ? 3.85 : 3.3;
+    const double per_block = full * (double)(nwg / 512) + (left == 0 ? 0.0 : left <= 256 ? half : most);
+    const double us = 6.0 + (double)(ntok < GM_BN ? ntok : GM_BN) / 64.0 + per_block * (double)mt_nsb(g) +
+                      1.6e-7 * (double)(g.rows * ntok);   // Y a little slower than there
+    // (a launch has fewer than 2^32 threads)
+    if (nwg >= ((int64_t)1 << 24) || 1.02 * us + 0.25 >= dense) return false;
+    *split_bytes = 0;
+    return true;
+}
+
 int64_t gemm_workspace_bytes(const lq_geom &g, int64_t ntok) {
-    const int64_t x = gemm_x_bytes(g, ntok), split = gemm_dense_split_bytes(g, ntok);
+    const int64_t x = gemm_x_bytes(g, ntok);
+    int64_t split = 0;
+    if (ntok > 0) gemm_takes_tile_kernel(g, ntok, &split);
     return split ? lq_align256(x) + split : x;
 }
 
@@ -762,7 +819,10 @@ int launch_gemm(const lq_geom &g, const uint8_t *W, const uint8_t *Wt, const flo
     const int64_t most = planes ? ntok : (((int64_t)1 << 32) - 1) / (2 * ldh);
     if (most < 1 || (planes && nwg > ((int64_t)1 << 30))) return fail(LOCALAI_EARG, "matmul: problem too large");
     if (int st = launch_x_to_f16(X, g.cols, g.cols, nullptr, 1, ntok, Xh, ldh, inv, s)) return st;
-    if (planes) return launch_gemm_t<GM_DENSE, GM_BN>(a, dim3((unsigned)((nwg + 7) / 8 * 8)), s);
+    const dim3 grid((unsigned)((nwg + 7) / 8 * 8));
+    if (planes) return launch_gemm_t<GM_DENSE, GM_BN>(a, grid, s);
+    int64_t split;
+    if (Wt && gemm_takes_tile_kernel(g, ntok, &split)) return launch_gemm_tile_t<GM_DENSE, GM_BN>(a, grid, s);
     const int64_t xb = lq_align256(gemm_x_bytes(g, ntok));
     for (int64_t t0 = 0; t0 < ntok;) {
         // (a tile has 128 tokens: all in one launch below 16.7 million columns)

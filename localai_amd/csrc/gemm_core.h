@@ -192,6 +192,6 @@ __device__ __forceinline__ lq_h8 gt_b(const GtRaw<T> &r, int q, uint32_t pair_ab
 // (Q5_K, Q4_0), a.Xh / a.inv filled in;
 // split_ws: up to split_bytes of scratch for K splits (none: one split)
 int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hipStream_t s);
-int64_t gemm_dense_split_bytes(const lq_geom &g, int64_t ntok);
+double gemm_dense_us(const lq_geom &g, int64_t ntok, int64_t *split_bytes);
 
 }  // namespace lq

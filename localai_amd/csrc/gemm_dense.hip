@@ -710,7 +710,26 @@ static DensePlan dense_plan(const lq_geom &g, int64_t ntok) {
     return p;
 }
 
-int64_t gemm_dense_split_bytes(const lq_geom &g, int64_t ntok) { return ntok < 1 ? 0 : dense_plan(g, ntok).bytes(); }
+// Time of a whole dense call (conversion of x included), for launch_gemm's choice
+// between this kernel and gemm_tile_kernel: fitted to 5900 calls (1 to 16 blocks
+// of K, 512 to 128256 rows, 1 to 2048 tokens; four in five within 5.5 %). Besides
+// the blocks, a workgroup's first loads and its stores are most of a short K's
+// time: 2048 x 768 Q4_K, 512 tokens, 32 workgroups: 20.5 us, of which the three
+// blocks take 9. *split_bytes: the parts' bytes.
+double gemm_dense_us(const lq_geom &g, int64_t ntok, int64_t *split_bytes) {
+    const DensePlan p = dense_plan(g, ntok);
+    *split_bytes = p.bytes();
+    const double fixed[4] = {6.1, 8.3, 9.2, 10.3}, block[4] = {1.6, 1.9, 2.3, 2.9};   // by computed MFMA tiles / 2
+    const int i = p.full || ntok > 96 ? 3 : (int)((ntok - 1) / 32), rounds = p.full / 256;
+    const double extra = g.type == LQ_Q6_K ? 0.3 : 0.0;                                 // more decode
+    double us = fixed[i];
+    if (rounds) us += (3.45 + extra) * (double)(rounds * gd_blocks(g)) + 2.4 * (double)(rounds - 1);
+    if (p.rest) us += (block[i] + extra) * (double)p.blocks + (rounds ? 2.6 : 0.0);
+    if (p.splits > 1)
+        us += 5.05 + 3.0 * (double)((p.splits - 1) / 8) +
+              (double)(p.rest * p.splits * (ntok < GD_BN ? ntok : GD_BN)) * GD_BM * 4.0 / 3.3e6;
+    return us;
+}
 
 int launch_gemm_dense(const GemmArgs &a, void *split_ws, int64_t split_bytes, hipStream_t s) {
     constexpr int lds = GD_RING * GD_SLOT;

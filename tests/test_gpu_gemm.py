@@ -237,6 +237,28 @@ def test_handles_without_the_tile_form(monkeypatch, t, rows, cols, tokens):
     check(out.T, raw, t, rows, cols, xs)
 
 
+@pytest.mark.parametrize('t', (12, 14, 8))
+@pytest.mark.parametrize('rows,nblocks,tokens', [(1, 1, 33), (16, 1, 40), (129, 3, 257), (300, 2, 130), (4112, 2, 2000)])
+def test_short_k_on_128_row_tiles(t, rows, nblocks, tokens):
+    """Products of few blocks of K, more than 32 tokens: the 128 x 128 tiles of the
+    tile form's older kernel. Ragged row and token edges, one to several
+    hundred workgroups, Q8_0 rows that end inside a block; no room for parts in
+    the workspace, both output layouts."""
+    from localai_amd import _lib, device
+    rng = np.random.default_rng(rows + 31 * nblocks + tokens + t)
+    cols = 256 * nblocks - (32 if t == 8 else 0)
+    raw = random_ggml(rng, t, rows * cols)
+    xs = rng.standard_normal((tokens, cols)).astype(np.float32)
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    least = (tokens + 15) // 16 * 16 * 256 * nblocks * 2 + tokens * 4
+    assert int(_lib.load().localai_hip_matmul_workspace_size(q.handle, tokens)) == least
+    xd = device.to_device_f32(xs)
+    got = q.matmul(xd).cpu().numpy()
+    check(got, raw, t, rows, cols, xs)
+    np.testing.assert_array_equal(q.matmul(xd, rows_major=True).cpu().numpy(), got.T)
+    q.close()
+
+
 @pytest.mark.parametrize('t', (2, 8))
 @pytest.mark.parametrize('cols', (32, 64, 96, 2144, 4128, 4192))
 def test_dense_rows_of_partial_blocks(t, cols):
