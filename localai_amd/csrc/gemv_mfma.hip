@@ -612,19 +612,30 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
     // one-vector plan; longer rows: 8 waves of ceil(nb / 8) blocks (up to 9 for
     // K <= 18432), which fit in registers only below 16 waves
     const int spw = nb <= 32 ? (nb + 15) / 16 : (nb + 7) / 8, waves = (nb + spw - 1) / spw;
-    // Row tiles per workgroup: a vector costs a wave about 82 instructions of
-    // staging and 35 a tile, and a CU one workgroup of 2 or 4 tiles at a time (two
-    // of one tile take as long as one after the other). More tiles share the
-    // staging as long as the workgroups still fill the CUs: 14336 x 4096 Q4_K, 31
-    // vectors: 1 tile 95.1 us, 2 65.2, 4 54.9; 4096 x 4096, 4 vectors: 7.0, 7.8,
-    // 12.2. Four tiles are left out for Q6_K (registers: 32000 rows, 7 vectors,
-    // 53.9 us against 49.5 with two) and below four vectors (14336 rows, 2
-    // vectors: 12.6 against 11.6), more than one where a wave has several blocks
-    // (4096 x 8192, 7 vectors: 24.4 against 16.0).
+    // Row tiles per workgroup (more than one only where a wave has one block:
+    // 4096 x 8192, 7 vectors 24.4 us with two, 16.0 with one). More tiles share the
+    // staging of x, as long as the workgroups still fill the CUs. The choice is the
+    // least of: a vector costs a wave 82 (staging) + 60 a tile on its SIMD, but a
+    // round of workgroups no less than 150 a tile (latency: one- to four-wave
+    // workgroups of four tiles leave the SIMDs idle); a CU holds 32 waves with one
+    // tile and, by registers and whole workgroups, 16 with two or four. Of 4101
+    // timed calls (1 to 16 blocks, 512 to 64000 rows, 2 to 31 vectors) 9 in 10 are
+    // within 4 % of the best choice, the mean 0.9 % off. 14336 x 4096 Q4_K, 31
+    // vectors: 1 tile 95.1 us, 2 65.2, 4 54.9; 4096 x 4096, 4 vectors: 7.0, 7.8, 12.2;
+    // 20000 x 1024, 5 vectors: 8.2, 7.5, 9.2; 10000 x 2304 Q6_K, 7 vectors: 13.7,
+    // 17.2. Four tiles are left out for Q6_K (registers: 32000 rows, 7 vectors, 53.9
+    // us against 49.5 with two) and for Q4_K below four vectors (14336 rows, 2
+    // vectors: 12.6 against 11.6).
     int rt = 1;
-    int64_t best = (tiles + 255) / 256 * (82 + 35);
-    for (int r = 2; spw == 1 && r <= (q6 || ntok < 4 ? 2 : 4); r *= 2) {
-        const int64_t cost = (tiles + 256 * r - 1) / (256 * r) * (82 + 35 * r);
+    int64_t best = INT64_MAX;
+    for (int r = 1; spw == 1 && r <= (q6 || (!q8 && ntok < 4) ? 2 : 4); r *= 2) {
+        const int64_t wgs = (tiles + r - 1) / r, per_cu = (wgs + 255) / 256;
+        const int64_t fit = (r == 1 ? 32 : 16) / nb > 1 ? (r == 1 ? 32 : 16) / nb : 1;
+        auto round = [&](int64_t n) {
+            const int64_t busy = (n * nb + 3) / 4 * (82 + 60 * r);
+            return n == 0 ? 0 : busy > 150 * r ? busy : (int64_t)(150 * r);
+        };
+        const int64_t cost = per_cu / fit * round(fit) + round(per_cu % fit);
         if (cost < best) {
             best = cost;
             rt = r;

@@ -124,7 +124,8 @@ def test_multi_vector_on_the_tile_form(t, rows, cols, ntok):
 
 @pytest.mark.parametrize('t', (12, 14, 8))
 @pytest.mark.parametrize('rows,nsb,ntok', [(16 * 260 - 3, 3, 6), (16 * 600 + 5, 2, 9), (16 * 780, 1, 31), (16 * 1100 + 1, 2, 4),
-                                           (40, 1, 13)])
+                                           (40, 1, 13), (16 * 900 - 3, 12, 5), (16 * 1000 - 9, 9, 7),
+                                           (16 * 1030 + 1, 10, 2)])
 def test_multi_vector_groups_and_row_tiles(t, rows, nsb, ntok):
     """Vector counts around the groups of four, one, two and four row tiles per
     workgroup, ragged last tiles: each y[t] equals the one-vector call bit
