@@ -95,7 +95,7 @@ def test_multi_vector(t, ntok):
 
 @pytest.mark.parametrize('t', (12, 14, 8))
 @pytest.mark.parametrize('rows,cols,ntok', [(200, 1024, 7), (14336, 4096, 3), (4096, 14336, 5), (300, 256 * 60, 2),
-                                            (48, 256 * 33, 4)])
+                                            (48, 256 * 33, 4), (200, 256 * 65, 9), (40, 256 * 72, 3)])
 def test_multi_vector_on_the_tile_form(t, rows, cols, ntok):
     """Several vectors through a Q4_K / Q6_K / Q8_0 handle run the tile-form
     kernel: every y[t] equals the one-vector call on x[t] bit for bit, the
