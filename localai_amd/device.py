@@ -42,12 +42,16 @@ def device():
 
 def stream_ptr(stream=None) -> int:
     """hipStream_t of `stream`, or of the current stream of the current device
-    (read directly: building the Stream object that current_stream() returns
-    took 2.8 us a call, a third of a small matvec's host time)."""
+    (read directly where PyTorch has the call: building the Stream object that
+    current_stream() returns took 2.8 us a call, a third of a small matvec's host
+    time; the call is not part of PyTorch's public interface)."""
     if stream is not None:
         return int(stream.cuda_stream)
     t = torch()
-    return t._C._cuda_getCurrentRawStream(t.cuda.current_device())
+    raw = getattr(t._C, '_cuda_getCurrentRawStream', None)
+    if raw is None:
+        return int(t.cuda.current_stream().cuda_stream)
+    return raw(t.cuda.current_device())
 
 
 def ptr(tensor) -> int:
