@@ -80,9 +80,9 @@ def test_k_lengths(t, nblocks):
 @pytest.mark.parametrize('rows,cols,tokens', [(112, 256, 256), (113, 512, 257), (300, 160, 300), (16, 768, 600),
                                             (1000, 1024, 512), (1800, 256, 256)])
 def test_q8_0_workgroup_tiles(rows, cols, tokens):
-    """Q8_0 with 256 tokens or more runs on 112-row x 256-token workgroup
-    tiles: ragged row and token edges, K padded up to whole 256-value blocks
-    (cols 160), one and several tiles each way, and both output layouts."""
+    """Q8_0 with 256 tokens or more: ragged row and token edges, K padded up to
+    whole 256-value blocks (cols 160), one and several tiles each way, and both
+    output layouts."""
     rng = np.random.default_rng(rows + cols + tokens)
     raw = random_ggml(rng, 8, rows * cols)
     xs = rng.standard_normal((tokens, cols)).astype(np.float32)
@@ -126,9 +126,9 @@ def test_dense_tiles_and_splits(t, rows, nblocks, tokens):
 @pytest.mark.parametrize('t,rows,nblocks,tokens', [(12, 4112, 3, 2000), (14, 4096, 2, 2048), (8, 3900, 4, 2100),
                                                    (13, 4112, 2, 2000), (2, 4100, 3, 1990)])
 def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
-    """More than 256 output tiles: whole rounds (a workgroup's next tile requested
-    before this one's results are stored), none or some tiles left over for
-    the split round, ragged edges; both output layouts hold the same values."""
+    """More than 256 output tiles of few blocks of K: one whole round, none or some
+    tiles left over (the Q4_K and Q8_0 shapes run the 128-row tile kernel), ragged
+    edges; both output layouts hold the same values."""
     rng = np.random.default_rng(rows + tokens)
     cols = 256 * nblocks
     raw = random_ggml(rng, t, rows * cols)
@@ -136,6 +136,37 @@ def test_dense_rounds_of_tiles(t, rows, nblocks, tokens):
     got = gpu_matmul(raw, t, rows, cols, xs)
     check(got, raw, t, rows, cols, xs)
     np.testing.assert_array_equal(gpu_matmul(raw, t, rows, cols, xs, rows_major=True), got.T)
+
+
+@pytest.mark.parametrize('t,nblocks', [(12, 10), (12, 11), (14, 10), (14, 11), (8, 10), (8, 11), (13, 6), (13, 7),
+                                       (2, 6), (2, 7)])
+@pytest.mark.parametrize('rows,tokens', [(8200, 2100), (8192, 2048)])
+def test_dense_two_rounds_and_parts(t, nblocks, rows, tokens):
+    """Two whole rounds of 256 tiles (a whole tile's first requests in flight while
+    the whole tile before it is stored), then 49 tiles in parts of K, which only
+    some workgroups have (561 tiles, ragged edges), or nothing (512 tiles); odd
+    and even block counts; every output against 64-bit products of the same
+    weights, in both layouts."""
+    from localai_amd import _lib, device
+    torch = device.torch()
+    rng = np.random.default_rng(t + nblocks + rows)
+    cols = 256 * nblocks
+    block, size = quant.block_layout(t)
+    part = np.frombuffer(random_ggml(rng, t, 257 * cols), np.uint8).reshape(-1, size)
+    raw = np.resize(part, (rows * cols // block, size)).tobytes()
+    q = device.QMat.from_ggml(raw, t, rows, cols)
+    least = (tokens + 15) // 16 * 16 * cols * 2 + tokens * 4
+    parts = int(_lib.load().localai_hip_matmul_workspace_size(q.handle, tokens)) - least
+    assert (parts >= 2 * 49 * 256 * 128 * 4) == (rows == 8200)
+    x = device.to_device_f32(rng.standard_normal((tokens, cols)))
+    got = q.matmul(x)
+    assert torch.equal(q.matmul(x, rows_major=True), got.T)
+    w, x = q.dequant().double().T.contiguous(), x.double()
+    ref = x @ w
+    err = (got.double() - ref).abs()
+    assert bool(err.le(MAX_REL * (x.abs() @ w.abs())).all())
+    assert float(err.max() / ref.abs().max()) < MAX_REL
+    q.close()
 
 
 @pytest.mark.parametrize('t,rows,cols,tokens', [(2, 3, (1 << 25) + 32, 66), (8, 3, (1 << 25) + 32, 66),
@@ -261,12 +292,13 @@ def test_short_k_on_128_row_tiles(t, rows, nblocks, tokens):
 
 @pytest.mark.parametrize('t', (2, 8))
 @pytest.mark.parametrize('cols', (32, 64, 96, 2144, 4128, 4192))
-def test_dense_rows_of_partial_blocks(t, cols):
+@pytest.mark.parametrize('tokens', (33, 20))
+def test_dense_rows_of_partial_blocks(t, cols, tokens):
     """32-value blocks: rows that end inside a 256-value block or a 64-value unit,
     around the 4096-value chunks of the row planes; the last block's scale is
     infinite in one row, whose outputs must not leak into others."""
     rng = np.random.default_rng(cols + t)
-    rows, tokens = 37, 33
+    rows = 37
     raw = random_ggml(rng, t, rows * cols)
     xs = rng.standard_normal((tokens, cols)).astype(np.float32)
     got = gpu_matmul(raw, t, rows, cols, xs)

@@ -1,7 +1,8 @@
 """The build-time check for kernels that count their own global loads
 (localai_amd/isa_check.py): planted hazards in small assembly listings must be
-found, correct waits must pass, and the GEMM kernel that relies on it must be
-clean in a fresh compile."""
+found, correct waits must pass, the kernels that rely on it must be clean in a
+fresh compile, and there, too, a wait made too lax by one must be found."""
+import re
 import shutil
 
 import pytest
@@ -153,3 +154,35 @@ def test_counted_load_kernels_are_clean(tmp_path):
             isa_check.check_source(build.HIPCC, build.COMMON, build.CSRC / src, kernel, tmp_path / 'k.s')
         else:
             isa_check.check_lds_ring(build.HIPCC, build.COMMON, build.CSRC / src, kernel, per_stage, tmp_path / 'k.s')
+
+
+@pytest.mark.skipif(shutil.which('hipcc') is None and not __import__('os').path.exists('/opt/rocm/bin/hipcc'),
+                    reason='hipcc not installed')
+def test_dense_gemm_wait_too_lax_by_one_is_found(tmp_path):
+    """The dense GEMM's four loops (2, 4, 6 and 8 MFMA tiles of tokens: 1 to 4 copies
+    of x a step and wave) share one ring check, with a bound of 4 copies from
+    before the last barrier. A step reads what was requested two barriers
+    earlier, so in each loop a wait that lets one more request stay in flight
+    leaves a copy two barriers old, or a block header that is decoded next: one
+    of the two checks finds it."""
+    from localai_amd import build
+    out = tmp_path / 'k.s'
+    isa_check.check_source(build.HIPCC, build.COMMON, build.CSRC / 'gemm_dense.hip', 'gemm_dense_kernel', out)
+    asm = out.read_text()
+    name = next(n for n in re.findall(r'^(_Z\S*gemm_dense_kernel\S*):', asm, re.M) if 'ILi12E' in n)
+    code = isa_check.kernel_lines(asm, name)
+    barriers = [i for i, l in enumerate(code) if l.startswith('s_barrier')]
+    planted, of_loop = 0, 0
+    for i in barriers:
+        # the step's wait: the last before its barrier, twice where a header comes too
+        j = next((k for k in range(i - 1, max(i - 60, 0), -1) if code[k].startswith('s_waitcnt vmcnt')), None)
+        n = 0 if j is None else int(re.search(r'vmcnt\((\d+)\)', code[j]).group(1))
+        of_loop = of_loop + 1 if 0 < n < 16 else 0
+        if not 1 <= of_loop <= 2:        # one step of each half in each loop
+            continue
+        lax = list(code)
+        for k in range(max(i - 60, 0), i):
+            lax[k] = lax[k].replace(f'vmcnt({n})', f'vmcnt({n + 1})')
+        assert isa_check.pending_violations(lax) or isa_check.lds_ring_violations(lax, 4), (i, code[j])
+        planted += 1
+    assert planted >= 2 * 4
