@@ -604,6 +604,31 @@ __device__ __forceinline__ void gt_main(const GemmArgs &a, _Float16 (*Xs)[BN * G
         const int64_t r0 = t0 * MT_ROWS + fr, r1 = t1 * MT_ROWS + fr;
         const bool ok0 = t0 < tiles && r0 < g.rows, ok1 = t1 < tiles && r1 < g.rows;
         float *yb0 = a.Y + p0 * a.y_ts + r0 * a.y_rs, *yb1 = a.Y + p0 * a.y_ts + r1 * a.y_rs;
+        if constexpr (MODE == GM_DENSE) {
+            // tokens contiguous: a lane's four in one store of four dwords, whatever
+            // their alignment (2048 x 768 Q4_K, 512 tokens: 22.4 -> 15.9 us)
+            if (a.y_ts == 1) {
+                typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const int lt = 16 * i + 4 * (lane >> 4);
+                    if (lt >= tn) continue;
+                    const lq_f4 sc = *reinterpret_cast<const lq_f4 *>(tsc + lt);
+                    const lq_f4 y0 = acc[i][0] * sc, y1 = acc[i][1] * sc;
+                    if (lt + 3 < tn) {
+                        if (ok0) *reinterpret_cast<f4u *>(yb0 + lt) = y0;
+                        if (ok1) *reinterpret_cast<f4u *>(yb1 + lt) = y1;
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 3; ++v) {
+                            if (ok0 && lt + v < tn) yb0[lt + v] = y0[v];
+                            if (ok1 && lt + v < tn) yb1[lt + v] = y1[v];
+                        }
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
 #pragma unroll
@@ -628,7 +653,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_tile_kernel(GemmArgs a) 
     constexpr int NI = BN / 16;            // 16-token MFMA tiles per wave
     constexpr int BB = mt_block_bytes(T);
     __shared__ __attribute__((aligned(16))) _Float16 Xs[2][BN * GM_BK];
-    __shared__ float tsc[BN];              // the output scale of each token of the tile
+    __shared__ __attribute__((aligned(16))) float tsc[BN];   // the output scale of each token of the tile
     __shared__ float asc[MODE == GM_MOE_GATE_UP ? BN : 1];   // gate_up with f16 output: its scale per token
     const lq_geom &g = a.g;
     // wave index made wave-uniform: row-tile addresses go to scalar registers
