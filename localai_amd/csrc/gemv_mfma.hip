@@ -562,7 +562,11 @@ __global__ __launch_bounds__(MAXT, MAXT == 1024 && SPW * RT == 1 ? 8 : 1) void g
     const MtLane<TYPE> L = mt_lane<TYPE>(lane);
     // do-while, at least one vector: with a test before the first pass the compiler
     // moved the loads behind it, between the weights' decoding of each block, and
-    // spilled (Q6_K, seven blocks a wave, 12288 x 14336, 2 vectors: 44.7 -> 48.9 us)
+    // spilled (Q6_K, seven blocks a wave, 12288 x 14336, 2 vectors: 44.7 -> 48.9 us).
+    // Q8_0 has no decoding to move, and keeps a test: without one the scales, loaded
+    // last and converted ahead of the loop, were waited for before the first x was
+    // staged (8192 x 15360, 2 vectors: 33.5 -> 35.6 us)
+    if (TYPE == LQ_Q8_0 && ntok < 1) return;
     int t0 = 0;
     do {
         const int nt = ntok - t0 < MT_TOKS ? ntok - t0 : MT_TOKS;
