@@ -732,12 +732,17 @@ static int64_t gemm_x_bytes(const lq_geom &g, int64_t ntok) {
 // 30.7; but 4096 x 4096, 128 tokens 26.9, 50.3 and 11008 x 2048, 300 tokens 34.5,
 // 39.0. Of 5160 calls up to 32000 rows the choice is within 4 % of the faster
 // kernel in all but 80, at worst 13 % off (11 % where it stays with the dense one).
-// Up to 32 tokens the dense kernel computes a quarter of what this one does.
+// Up to 32 tokens the dense kernel computes a quarter of what this one does, except
+// from 256 of its tiles on, where it computes whole ones: of 882 calls of 66000 to
+// 256000 rows and up to 128 tokens, 25 are more than 4 % off the faster kernel
+// (128256 x 1536 Q8_0, 32 tokens 57.0 us dense, 55.5 here; 202048 x 768, 1 token
+// 53.7, 45.4).
 // (The tile kernel's offsets into Y have 32 bits.)
 // *split_bytes: what the parts of K of the dense kernel take, 0 with the tile kernel.
 static bool gemm_takes_tile_kernel(const lq_geom &g, int64_t ntok, int64_t *split_bytes) {
     const double dense = gemm_dense_us(g, ntok, split_bytes);
-    if (mt_matrix_bytes(g) == 0 || ntok <= 32 || g.rows >= ((int64_t)1 << 25)) return false;
+    const bool rounds = (g.rows + 255) / 256 * ((ntok + 127) / 128) >= 256;
+    if (mt_matrix_bytes(g) == 0 || (ntok <= 32 && !rounds) || g.rows >= ((int64_t)1 << 25)) return false;
     const int64_t nwg = ((g.rows + GM_BM - 1) / GM_BM) * ((ntok + GM_BN - 1) / GM_BN), left = nwg % 512;
     // us per block: a full round of 512 workgroups, one of up to 256, of more
     const double full = g.type == LQ_Q4_K ? 3.75 : g.type == LQ_Q6_K ? 4.15 : 3.9;

@@ -725,6 +725,8 @@ double gemm_dense_us(const lq_geom &g, int64_t ntok, int64_t *split_bytes) {
     double us = fixed[i];
     if (rounds) us += (3.45 + extra) * (double)(rounds * gd_blocks(g)) + 2.4 * (double)(rounds - 1);
     if (p.rest) us += (block[i] + extra) * (double)p.blocks + (rounds ? 2.6 : 0.0);
+    // one token tile: every weight of the rounds comes from memory, and Q8_0 has most
+    if (rounds && ntok <= GD_BN && g.type == LQ_Q8_0) us += 0.3 * (double)((rounds + (p.rest ? 1 : 0)) * gd_blocks(g));
     if (p.splits > 1)
         us += 5.05 + 3.0 * (double)((p.splits - 1) / 8) +
               (double)(p.rest * p.splits * (ntok < GD_BN ? ntok : GD_BN)) * GD_BM * 4.0 / 3.3e6;

@@ -269,10 +269,11 @@ def test_handles_without_the_tile_form(monkeypatch, t, rows, cols, tokens):
 
 
 @pytest.mark.parametrize('t', (12, 14, 8))
-@pytest.mark.parametrize('rows,nblocks,tokens', [(1, 1, 33), (16, 1, 40), (129, 3, 257), (300, 2, 130), (4112, 2, 2000)])
+@pytest.mark.parametrize('rows,nblocks,tokens', [(1, 1, 33), (16, 1, 40), (129, 3, 257), (300, 2, 130), (4112, 2, 2000),
+                                                 (81001, 1, 5)])
 def test_short_k_on_128_row_tiles(t, rows, nblocks, tokens):
-    """Products of few blocks of K, more than 32 tokens: the 128 x 128 tiles of the
-    tile form's older kernel. Ragged row and token edges, one to several
+    """Products of few blocks of K, more than 32 tokens (or very many rows): the 128 x
+    128 tiles of the tile form's older kernel. Ragged row and token edges, one to several
     hundred workgroups, Q8_0 rows that end inside a block; no room for parts in
     the workspace, both output layouts."""
     from localai_amd import _lib, device
