@@ -92,11 +92,14 @@ int localai_hip_ggml_matvec(int ggml_type, const void *w_dev, int64_t rows, int6
  * Q4_0, Q8_0, Q4_K, Q5_K, Q6_K (the reference's native types,
  * engine/native_quant.py:104). cols must be a multiple of the block size.
  * Q4_K, Q6_K and Q8_0 handles hold the MFMA tile form only (the same bytes
- * as GGML, reordered); the row-plane form that the several-vector matvec,
- * the Q8_0 matvec of rows that are not whole 256-value super-blocks and the
- * fallback MoE paths read is built from it on the first such call (which
- * allocates and waits for the stream, so not under graph capture:
- * LOCALAI_ESTATE there) and then kept. Other types hold the row planes.
+ * as GGML, reordered); the row-plane form that the matvecs of rows outside
+ * the MFMA matvec's range (Q8_0 rows that are not whole 256-value
+ * super-blocks, rows of more than 72 of them) and the fallback MoE paths read
+ * is built from it on the first such call (which allocates and waits for the
+ * stream, so not under graph capture: LOCALAI_ESTATE there) and then kept.
+ * Other types hold the row planes, as every type does in a handle made while
+ * the environment has LOCALAI_HIP_MFMA_MATVEC=0: the row-plane kernels then
+ * serve all of its calls.
  * With the tile form a handle also keeps, per matrix, the largest row L2
  * norm of its first and of its second half of rows (8 bytes per matrix;
  * the prefill MoE gate_up GEMM scales its f16 outputs from them). */
@@ -148,8 +151,13 @@ int localai_hip_matvec_many(int n, const localai_qmat *const *mats, const int64_
  * converted rows and, where few output tiles leave room on the chip, partial
  * sums of a division of K. A workspace with room for the converted rows only
  * (tokens rounded up to 16, times cols rounded up to 256, 2 bytes each, plus 4
- * bytes a token) is accepted too: K is then divided less (the sums are taken
- * in another order). */
+ * bytes a token) is accepted too: K is then divided less.
+ * How K is divided follows from the matrix's shape and type, the token count and
+ * the workspace, and within one call the output tiles left over after whole
+ * rounds of 256 are divided where the others are not. So a call's results are
+ * reproducible for the same shape, token count and workspace size (in both
+ * layouts), but a token's are not bit-equal across token counts: their fp32
+ * partial sums add up in another order (about 1e-7 of sum |w x|). */
 int64_t localai_hip_matmul_workspace_size(const localai_qmat *m, int64_t tokens);
 
 /* Many-token product with matrix `expert` of the handle; counterpart of

@@ -1,5 +1,6 @@
-// Dense prefill product on f16 MFMA: the kernel that every dense matmul runs
-// (contract and arithmetic: gemm.hip).
+// Dense prefill product on f16 MFMA: the kernel of all dense matmuls but those of
+// short K and of handles without the tile form (gemm.hip, which also has the
+// contract and the arithmetic).
 //
 // Workgroup: 8 waves x 2 row tiles (256 weight rows) x 128 tokens (16 NV of
 // them computed), over a range of 256-value blocks of K. Each wave decodes its
@@ -10,7 +11,8 @@
 // overlaps: a 32-value slice of a wave is 2 NV MFMAs (16 clocks each), 28 to
 // 60 VALU of decode and NV LDS reads, and run one after the other they took
 // 4.8 us per 256 x 128 x 256 block against 1.9 us of MFMAs. Simple VALU issues
-// under a running MFMA (16 MFMAs alone 112.7 ns, with 32 v_and 110.7 ns), so
+// under a running MFMA (16 MFMAs alone 108 to 113 ns, with 32 v_and, v_perm or f32
+// multiply-adds 115 to 121 ns), so
 // every slice's MFMAs are interleaved with the reads and the decode of the
 // next slice, across the workgroup barrier too:
 //   step s (128 values), slices kk = 0 .. 3: MFMAs of slice kk, beside them
@@ -307,9 +309,9 @@ struct GdMain {
             }
             return;
         } else {
-        const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
-        gd_load_step<T, HALF>(d[0], w0p + o, l16);
-        gd_load_step<T, HALF>(d[1], w1p + o, l16);
+            const int64_t o = (int64_t)(b < nb ? b : nb - 1) * BB;
+            gd_load_step<T, HALF>(d[0], w0p + o, l16);
+            gd_load_step<T, HALF>(d[1], w1p + o, l16);
         }
     }
     __device__ __forceinline__ void load_block(GdBlock<T> (&d)[2], int b) {
@@ -682,7 +684,8 @@ struct DensePlan {
 // or 3.2 (128: bound by its MFMAs and decode, the others by latency), while parts
 // write and read their sums (3.5 TB/s for both ways together) and need the
 // summing launch (5 us, 1.5 more for every further eight parts it adds up): the
-// split with the least total. Measured, whole calls: 4096 x 4096 Q4_K, 77 tokens:
+// split with the least total. One set of constants for all types, from Q4_K and
+// Q6_K calls (Q5_K's decode takes longer per block). Measured, whole calls: 4096 x 4096 Q4_K, 77 tokens:
 // 1 part 49.6 us, 4 23.8, 8 (taken) 22.3, 16 25.2; 14336 x 4096, 256 tokens: 1
 // 56.9, 2 (taken) 45.8; 4096 x 14336 Q6_K, 333 tokens: 1 183, 4 64.8, 5 (taken)
 // 63.9, 8 98 (two rounds); 14080 x 1280, 120 tokens: 1 (taken) 25.3, 3 26.9.

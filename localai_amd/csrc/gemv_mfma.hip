@@ -541,9 +541,9 @@ __host__ __device__ constexpr size_t mt_tok_lds_bytes(int type, int waves, int s
 }
 
 template <int TYPE, int SPW, int RT, int MAXT>
-__global__ __launch_bounds__(MAXT, MAXT == 1024 && SPW * RT == 1 ? 8 : 1) void gemv_mfma_tok(const uint8_t *__restrict__ Wt, int64_t rows, int nb,
-                                                      int64_t tiles, const float *__restrict__ x, int64_t ldx,
-                                                      float *__restrict__ y, int64_t ldy, int ntok) {
+__global__ __launch_bounds__(MAXT, MAXT == 1024 && SPW * RT == 1 ? 8 : 1)
+void gemv_mfma_tok(const uint8_t *__restrict__ Wt, int64_t rows, int nb, int64_t tiles, const float *__restrict__ x,
+                   int64_t ldx, float *__restrict__ y, int64_t ldy, int ntok) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int XB = mt_xbytes(TYPE);
     const int lane = lane_id(), wv = wave_id(), nw = blockDim.x >> 6, sb0 = wv * SPW, nsb = mt_nsb(nb, sb0, SPW);
@@ -642,7 +642,8 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
     // 20000 x 1024, 5 vectors: 8.2, 7.5, 9.2; 10000 x 2304 Q6_K, 7 vectors: 13.7,
     // 17.2. Four tiles are left out for Q6_K (registers: 32000 rows, 7 vectors, 53.9
     // us against 49.5 with two) and for Q4_K below four vectors (14336 rows, 2
-    // vectors: 12.6 against 11.6).
+    // vectors: 12.6 against 11.6). Four Q4_K tiles are at the limit of 128 registers
+    // and spill ten, Q8_0's take 126.
     int rt = 1;
     int64_t best = INT64_MAX;
     for (int r = 1; spw == 1 && r <= (q6 || (!q8 && ntok < 4) ? 2 : 4); r *= 2) {
@@ -682,7 +683,7 @@ int launch_matvec_mfma_tok(const lq_geom &g, const uint8_t *Wt, const float *x, 
             else if (rt == 2) MT_T(1, 2, 1024);
             else MT_T(1, 1, 1024);
             break;
-                case 2: MT_T(2, 1, 1024); break;
+        case 2: MT_T(2, 1, 1024); break;
         case 5: MT_T(5, 1, 512); break;
         case 6: MT_T(6, 1, 512); break;
         case 7: MT_T(7, 1, 512); break;
